@@ -18,9 +18,10 @@
 //     wide: as project_rows_kernel<1>, with the input row staged once per
 //     workgroup in LDS (requested ahead of the weights) instead of read from
 //     L2 by every wave.
-//   project_tiles_kernel: many tokens (prompt). MFMA-bound: 128 x 128 output
-//     tiles, 32-column K steps double-buffered in LDS as f32, the products on
-//     v_mfma_f64_16x16x4f64 after converting the operands to f64.
+//   project_tiles_kernel: more than 16 tokens (prompt). MFMA-bound: output
+//     tiles of 128 x 128 down to 32 x 32, K steps double-buffered in LDS as
+//     f32, the products on v_mfma_f64_16x16x4f64 after converting the
+//     operands to f64.
 //   post_norm_kernel: one workgroup per token: the row's f64 sum of squares
 //     (per-thread partial sums, then a fixed tree of lane shuffles and the
 //     four waves), inv = 1/sqrt(ms + eps) in f64, y = f32(x * inv) * scale,
@@ -29,9 +30,17 @@
 #include "context.hpp"
 #include "pcl_attention.h"
 
+#include <algorithm>
+#include <atomic>
 #include <cstdio>
+#include <iterator>
+#include <utility>
 
 namespace pcl {
+
+constexpr int kMaxDevices = 64;
+
+int device_cus();
 
 constexpr int kErrBlock = 8; // non-finite value in the output block
 
@@ -47,7 +56,10 @@ struct BlockParams {
     int *err;
 };
 
-constexpr int kRowTokens = 16; // tokens per pass of the row kernel
+// Largest token count of the row kernel: 16 tokens run 55 us there and 66 us
+// in tiles (2816 x 4096), 17-32 tokens took it two passes (24 tokens 108 us,
+// in tiles 67 us).
+constexpr int kRowTokens = 16;
 
 // One wave per output row; tokens [t0, t0 + min(NT, n - t0)) per launch
 // pass. Instantiated for NT = 1, 2, 4, 8 and 16: a one-token decode then
@@ -128,38 +140,48 @@ __global__ __launch_bounds__(256) void project_rows_kernel(BlockParams p, int t0
     }
 }
 
-// 128 x 128 output tile per 256-thread workgroup (2 x 2 waves of 64 x 64),
-// K in steps of 32 columns, LDS rows padded to 36 floats (16-byte aligned,
-// and the 16 rows an MFMA operand read touches fall in distinct banks).
-constexpr int kTileM = 128, kTileN = 128, kTileK = 32, kLdsRow = 36;
-
+// TM x TN output tile per 256-thread workgroup (2 x 2 waves of TM/2 x TN/2),
+// K in steps of TK columns, LDS rows padded by 4 floats (16-byte aligned, and
+// the 16 rows an MFMA operand read touches fall in distinct banks). Every
+// output sums its columns in the same order in every instantiation.
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-// Two workgroups per CU (2 x 72 KiB of LDS; registers held to 256 per lane,
-// which also keeps the f64 accumulators out of AGPRs): 16 % faster than one
-// on a 4K-token projection, where the other workgroup hides a wave's LDS and
-// conversion latency between MFMAs.
+template <int TM, int TN, int TK>
+constexpr size_t tile_lds_bytes()
+{
+    return 2 * sizeof(float) * (TM + TN) * (TK + 4);
+}
+
+// Two workgroups per CU (at most 2 x 72 KiB of LDS; registers held to 256
+// per lane, which also keeps the f64 accumulators out of AGPRs): 16 % faster
+// than one on a 4K-token projection, where the other workgroup hides a
+// wave's LDS and conversion latency between MFMAs.
+template <int TM, int TN, int TK>
 __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
 {
-    __shared__ __attribute__((aligned(16))) float sa[2][kTileM * kLdsRow];
-    __shared__ __attribute__((aligned(16))) float sb[2][kTileN * kLdsRow];
+    constexpr int kRow = TK + 4;
+    constexpr int kQuads = TK / 4;              // float4 per row and K step
+    constexpr int kLoadA = TM * kQuads / 256;   // float4 per thread and K step
+    constexpr int kLoadB = TN * kQuads / 256;
+    constexpr int kI = TM / 32, kJ = TN / 32;   // 16 x 16 blocks of a wave
+    extern __shared__ __attribute__((aligned(16))) float tiles[];
+    // two buffers of A rows, then two of B rows
+    float *const sa = tiles, *const sb = tiles + 2 * TM * kRow;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const int m0 = blockIdx.y * kTileM, n0 = blockIdx.x * kTileN;
+    const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
+    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
 
-    // global -> registers -> LDS: each thread moves 4 float4 of A and 4 of B
-    // per K step; the next step's loads are in flight during this step's MFMAs
-    f4 ra[4], rb[4];
+    // global -> registers -> LDS; the next step's loads are in flight during
+    // this step's MFMAs
+    f4 ra[kLoadA], rb[kLoadB];
     auto load = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + 256 * i; // row = idx / 8, quad = idx % 8
-            const int row = idx >> 3, q = idx & 7;
-            const int k = k0 + 4 * q;
+        for (int i = 0; i < kLoadA; ++i) {
+            const int idx = tid + 256 * i;
+            const int row = idx / kQuads, k = k0 + 4 * (idx % kQuads);
             ra[i] = f4{0.f, 0.f, 0.f, 0.f};
-            rb[i] = f4{0.f, 0.f, 0.f, 0.f};
             if (m0 + row < p.n) {
                 const float *src = p.x + (int64_t)(m0 + row) * p.in;
                 if (k + 3 < p.in)
@@ -168,6 +190,12 @@ __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
                     for (int e = 0; e < 4; ++e)
                         ra[i][e] = k + e < p.in ? ldg(src + k + e) : 0.f;
             }
+        }
+#pragma unroll
+        for (int i = 0; i < kLoadB; ++i) {
+            const int idx = tid + 256 * i;
+            const int row = idx / kQuads, k = k0 + 4 * (idx % kQuads);
+            rb[i] = f4{0.f, 0.f, 0.f, 0.f};
             if (n0 + row < p.out) {
                 const float *src = p.w + (int64_t)(n0 + row) * p.in;
                 if (k + 3 < p.in)
@@ -180,22 +208,25 @@ __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
     };
     auto store = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < kLoadA; ++i) {
             const int idx = tid + 256 * i;
-            const int row = idx >> 3, q = idx & 7;
-            *(f4 *)(sa[buf] + row * kLdsRow + 4 * q) = ra[i];
-            *(f4 *)(sb[buf] + row * kLdsRow + 4 * q) = rb[i];
+            *(f4 *)(sa + buf * TM * kRow + idx / kQuads * kRow + 4 * (idx % kQuads)) = ra[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kLoadB; ++i) {
+            const int idx = tid + 256 * i;
+            *(f4 *)(sb + buf * TN * kRow + idx / kQuads * kRow + 4 * (idx % kQuads)) = rb[i];
         }
     };
 
-    d4 acc[4][4];
+    d4 acc[kI][kJ];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kI; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < kJ; ++j)
             acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
 
-    const int steps = (p.in + kTileK - 1) / kTileK;
+    const int steps = (p.in + TK - 1) / TK;
     load(0);
     store(0);
     __syncthreads();
@@ -203,22 +234,23 @@ __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
     for (int s = 0; s < steps; ++s) {
         const int buf = s & 1;
         if (s + 1 < steps)
-            load((s + 1) * kTileK);
+            load((s + 1) * TK);
 #pragma unroll
-        for (int kc = 0; kc < kTileK; kc += 16) {
+        for (int kc = 0; kc < TK; kc += 16) {
             // MFMA k slot kq of step j holds column kc + 4 kq + j
-            f4 a[4], b[4];
+            f4 a[kI], b[kJ];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = *(const f4 *)(sa[buf] + (wm + 16 * i + r16) * kLdsRow + kc + 4 * kq);
-                b[i] = *(const f4 *)(sb[buf] + (wn + 16 * i + r16) * kLdsRow + kc + 4 * kq);
-            }
+            for (int i = 0; i < kI; ++i)
+                a[i] = *(const f4 *)(sa + (buf * TM + wm + 16 * i + r16) * kRow + kc + 4 * kq);
+#pragma unroll
+            for (int i = 0; i < kJ; ++i)
+                b[i] = *(const f4 *)(sb + (buf * TN + wn + 16 * i + r16) * kRow + kc + 4 * kq);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < kI; ++i)
 #pragma unroll
-                    for (int jj = 0; jj < 4; ++jj)
+                    for (int jj = 0; jj < kJ; ++jj)
                         acc[i][jj] = __builtin_amdgcn_mfma_f64_16x16x4f64(
                             (double)a[i][j], (double)b[jj][j], acc[i][jj], 0, 0, 0);
         }
@@ -229,14 +261,14 @@ __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
     // acc[i][jj][e]: row wm + 16i + kq + 4e, column wn + 16 jj + r16 (the f64
     // MFMA's output rows interleave by lane group, unlike the f32 one's)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kI; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int row = m0 + wm + 16 * i + kq + 4 * e;
             if (row >= p.n)
                 continue;
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
+            for (int jj = 0; jj < kJ; ++jj) {
                 const int col = n0 + wn + 16 * jj + r16;
                 if (col < p.out)
                     stg(p.proj + (int64_t)row * p.out + col, (float)acc[i][jj][e]);
@@ -386,28 +418,83 @@ __global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p, int
         stg(p.proj + (int64_t)t0 * p.out + r, (float)acc);
 }
 
+template <int TM, int TN, int TK>
+static hipError_t launch_tile(const BlockParams &p, hipStream_t stream)
+{
+    constexpr size_t lds = tile_lds_bytes<TM, TN, TK>();
+    static std::atomic<bool> configured[kMaxDevices];
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess)
+        return e;
+    if (dev < 0 || dev >= kMaxDevices)
+        return hipErrorInvalidDevice;
+    if (!configured[dev].load(std::memory_order_acquire)) {
+        e = hipFuncSetAttribute((const void *)project_tiles_kernel<TM, TN, TK>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess)
+            return e;
+        configured[dev].store(true, std::memory_order_release);
+    }
+    const dim3 grid((p.out + TN - 1) / TN, (p.n + TM - 1) / TM);
+    project_tiles_kernel<TM, TN, TK><<<grid, 256, lds, stream>>>(p);
+    return hipGetLastError();
+}
+
+// The tile with the least time by tiles per CU: the CU with the most tiles
+// sets it, so 352 tiles of 128 x 128 (2000 tokens, 2816 rows) cost two
+// rounds for 1.4 rounds of work, and a few tokens leave most CUs idle under
+// large tiles, while small ones reach a lower MFMA rate. The constants are
+// measured (4096 columns, one MI355X, us): a tile's share of its CU's time,
+// and the fill and drain of a launch. Projection of 2816 rows, 128 x 128
+// alone against the chosen tile: 33 tokens 568 -> 67 us, 256 tokens 578 ->
+// 152 us, 1000 tokens 590 -> 468 us, 2000 tokens 1080 -> 868 us; 4096 tokens
+// keep 128 x 128 (1.61 ms, 0.74 of the fp64 MFMA peak).
+static hipError_t launch_tiles(const BlockParams &p, hipStream_t stream)
+{
+    const int64_t cus = std::max(device_cus(), 1);
+    auto cost = [&](int tm, int tn, int fixed, int per_tile) {
+        const int64_t tiles = (int64_t)((p.out + tn - 1) / tn) * ((p.n + tm - 1) / tm);
+        return fixed + (tiles + cus - 1) / cus * per_tile;
+    };
+    using Launch = hipError_t (*)(const BlockParams &, hipStream_t);
+    const std::pair<int64_t, Launch> tiles[] = {
+        {cost(128, 128, 45, 515), launch_tile<128, 128, 32>},
+        {cost(128, 64, 40, 281), launch_tile<128, 64, 32>},
+        {cost(64, 64, 25, 147), launch_tile<64, 64, 64>},
+        {cost(64, 32, 33, 77), launch_tile<64, 32, 64>},
+        {cost(32, 32, 10, 44), launch_tile<32, 32, 128>},
+    };
+    // past 8192 tiles of 128 x 128 (32 rounds) a last round is a few percent,
+    // and the grids of smaller tiles could leave the launch limits (65535
+    // blocks of rows)
+    const bool many = ((p.out + 127) / 128) * (int64_t)((p.n + 127) / 128) > 8192;
+    const auto least = std::min_element(
+        std::begin(tiles), many ? std::begin(tiles) + 1 : std::end(tiles),
+        [](const auto &a, const auto &b) { return a.first < b.first; });
+    return least->second(p, stream);
+}
+
 hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
 {
-    if (p.n <= 2 * kRowTokens) {
+    if (p.n <= kRowTokens) {
         const dim3 grid((p.out + 3) / 4);
-        for (int t0 = 0; t0 < p.n; t0 += kRowTokens) {
-            const int nt = p.n - t0 < kRowTokens ? p.n - t0 : kRowTokens;
-            if (nt == 1 && p.in % 4 == 0 && p.in <= kLdsRowFloats)
-                project_row_lds_kernel<<<grid, 256, p.in * 4, stream>>>(p, t0);
-            else if (nt == 1)
-                project_rows_kernel<1><<<grid, 256, 0, stream>>>(p, t0);
-            else if (nt == 2)
-                project_rows_kernel<2><<<grid, 256, 0, stream>>>(p, t0);
-            else if (nt <= 4)
-                project_rows_kernel<4><<<grid, 256, 0, stream>>>(p, t0);
-            else if (nt <= 8)
-                project_rows_kernel<8><<<grid, 256, 0, stream>>>(p, t0);
-            else
-                project_rows_kernel<16><<<grid, 256, 0, stream>>>(p, t0);
-        }
+        if (p.n == 1 && p.in % 4 == 0 && p.in <= kLdsRowFloats)
+            project_row_lds_kernel<<<grid, 256, p.in * 4, stream>>>(p, 0);
+        else if (p.n == 1)
+            project_rows_kernel<1><<<grid, 256, 0, stream>>>(p, 0);
+        else if (p.n == 2)
+            project_rows_kernel<2><<<grid, 256, 0, stream>>>(p, 0);
+        else if (p.n <= 4)
+            project_rows_kernel<4><<<grid, 256, 0, stream>>>(p, 0);
+        else if (p.n <= 8)
+            project_rows_kernel<8><<<grid, 256, 0, stream>>>(p, 0);
+        else
+            project_rows_kernel<16><<<grid, 256, 0, stream>>>(p, 0);
     } else {
-        const dim3 grid((p.out + kTileN - 1) / kTileN, (p.n + kTileM - 1) / kTileM);
-        hipLaunchKernelGGL(project_tiles_kernel, grid, dim3(256), 0, stream, p);
+        const hipError_t e = launch_tiles(p, stream);
+        if (e != hipSuccess)
+            return e;
     }
     hipLaunchKernelGGL(post_norm_kernel, dim3(p.n), dim3(256), 0, stream, p);
     return hipGetLastError();

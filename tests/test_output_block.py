@@ -78,11 +78,11 @@ def run_block(torch, ctx, x, w, scale, res, eps=1e-6, in_place=False):
     return proj.cpu().numpy(), out.cpu().numpy(), err
 
 
-# n = 1, 5, 16, 32: row streaming; 33, 200, 300: f64 MFMA tiles. One token
+# n = 1, 5, 7, 16: few tokens; 17, 32, 33, 200, 300: f64 MFMA tiles. One token
 # with input rows of at most 16384 columns (a multiple of 4) is projected
 # with the input row staged in LDS: rows of 1000 (fewer than 4096 columns),
 # 5000 (4096 and a partial step), 4000 (one 4096-column step taken by some
-# lanes only) and 4096 columns, the last token of 17; 16388 and 1001
+# lanes only) and 4096 columns; 16388 and 1001
 # columns take the plain one-token kernel.
 BLOCK_CASES = [(1, 4096, 2816), (5, 4096, 2816), (16, 8192, 2816), (32, 4096, 1536),
                (33, 4096, 2816), (200, 4096, 300), (300, 1000, 130), (7, 1001, 77),
@@ -110,6 +110,33 @@ def test_output_block_matches_the_oracle(torch, ctx, oracle, case):
         assert np.max(np.abs(out[t] - want)) <= 1e-5
         same += int(np.sum(proj[t].view(np.uint32) == want_p.view(np.uint32)))
     assert same >= 0.999 * n * rows
+
+
+# 17-40 tokens: 32 x 32 tiles, one and two blocks of rows with remainders;
+# 520 x 2816: 64 x 32 or 64 x 64; 530 tokens over 4220 rows: 128 x 64; 1400
+# over 2816: 128 x 128 (the choice follows the device's CU count). Columns
+# below, at and past each K step, and not a multiple of 4.
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [(17, 127, 33), (31, 128, 32), (40, 130, 65), (129, 66, 2816),
+                                  (520, 65, 2816), (700, 63, 2816), (530, 34, 4220),
+                                  (1400, 31, 2816)], ids=lambda c: "x".join(map(str, c)))
+def test_projection_tiles_match_f64_sums(torch, ctx, case):
+    n, cols, rows = case
+    g = np.random.default_rng(sum(case))
+    x = g.standard_normal((n, cols)).astype(np.float32)
+    w = (g.standard_normal((rows, cols)) / np.sqrt(cols)).astype(np.float32)
+    scale = (1 + 0.1 * g.standard_normal(rows)).astype(np.float32)
+    res = g.standard_normal((n, rows)).astype(np.float32)
+    proj, out, err = run_block(torch, ctx, x, w, scale, res)
+    assert err == 0
+    p64 = x.astype(np.float64) @ w.astype(np.float64).T
+    # one rounding to f32, and f64 sums of `cols` terms in another order
+    slack = 2.0 ** -24 * np.abs(p64) + cols * 2.0 ** -52 * (np.abs(x).astype(np.float64)
+                                                            @ np.abs(w).astype(np.float64).T)
+    assert np.all(np.abs(proj - p64) <= slack)
+    q64 = proj.astype(np.float64)
+    want = res + (q64 / np.sqrt(np.mean(q64 * q64, axis=1, keepdims=True) + 1e-6)) * scale
+    assert np.max(np.abs(out - want)) <= 1e-5
 
 
 @pytest.mark.gpu
