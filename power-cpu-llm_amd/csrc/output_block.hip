@@ -10,7 +10,8 @@
 // the two f64 sums straddle an f32 rounding boundary, and a sum like
 // 2^24 + 1 - 2^24 stays exact.
 //
-//   project_rows_kernel: few tokens (decode, verification). HBM-bound on the
+//   project_rows_kernel: one or two tokens (up to 16 where the columns are
+//     not whole 16-byte quads). HBM-bound on the
 //     weights: one wave per output row streams the row once with 16-byte
 //     loads, 4096 columns in flight at a time, and keeps one f64 accumulator
 //     per token per lane; the tokens' inputs come from L2.
@@ -18,7 +19,10 @@
 //     wide: as project_rows_kernel<1>, with the input row staged once per
 //     workgroup in LDS (requested ahead of the weights) instead of read from
 //     L2 by every wave.
-//   project_tiles_kernel: more than 16 tokens (prompt). MFMA-bound: output
+//   project_few_kernel: 3 to 64 tokens (verification, short prompts; 128 for
+//     few output rows): the waves of a workgroup split the columns of 16
+//     output rows, f64 MFMAs on operands loaded straight from memory.
+//   project_tiles_kernel: more tokens (prompt). MFMA-bound: output
 //     tiles of 128 x 128 down to 32 x 32, K steps double-buffered in LDS as
 //     f32, the products on v_mfma_f64_16x16x4f64 after converting the
 //     operands to f64.
@@ -56,9 +60,9 @@ struct BlockParams {
     int *err;
 };
 
-// Largest token count of the row kernel: 16 tokens run 55 us there and 66 us
-// in tiles (2816 x 4096), 17-32 tokens took it two passes (24 tokens 108 us,
-// in tiles 67 us).
+// Largest token count of the row kernel (columns that are not whole 16-byte
+// quads; else two tokens): 16 tokens run 55 us there and 66 us in tiles (2816
+// x 4096), 17-32 tokens took it two passes (24 tokens 108 us, in tiles 67 us).
 constexpr int kRowTokens = 16;
 
 // One wave per output row; tokens [t0, t0 + min(NT, n - t0)) per launch
@@ -418,6 +422,98 @@ __global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p, int
         stg(p.proj + (int64_t)t0 * p.out + r, (float)acc);
 }
 
+// 16 output rows x 16 NB tokens per workgroup, its eight waves splitting the
+// columns: 32-column pieces go round the waves (256 columns, 1 KiB of a row,
+// per step). Bound by the weights' stream and its round trips: a wave loads
+// MFMA operands straight from memory (every weight is used by one wave only,
+// so LDS would add a pass), one piece requested ahead of the piece being
+// multiplied (two or four ahead were slower, 16 tokens 24.2 against 24.5 and
+// 27.3 us). The waves' f64 sums meet in LDS and are added in wave order.
+// p.in % 4 == 0. Projection of 2816 x 4096 with its post-norm, one wave per
+// row (in tiles past 16 tokens) against this: 4 tokens 22.9 -> 19.1 us, 16
+// tokens 53 -> 24.2 us, 32 tokens 66 -> 31.9 us, 64 tokens 69 -> 50.9 us.
+constexpr int kFewWaves = 8;
+constexpr int kFewStep = 32 * kFewWaves; // columns per piece of all waves
+
+template <int NB>
+__global__ __launch_bounds__(64 * kFewWaves, 2) void project_few_kernel(BlockParams p)
+{
+    __shared__ double sums[kFewWaves][NB * 256];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int r16 = lane & 15, kq = lane >> 4;
+    const int r0 = blockIdx.x * 16, t0 = blockIdx.y * 16 * NB;
+    const int c0 = 32 * wave + 8 * kq; // this lane's first column of piece 0
+    // rows and tokens past the last repeat it (not written)
+    const float *wr = p.w + (int64_t)min(r0 + r16, p.out - 1) * p.in;
+    const float *xr[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        xr[b] = p.x + (int64_t)min(t0 + 16 * b + r16, p.n - 1) * p.in;
+
+    struct Piece {
+        f4 w[2], x[NB][2];
+    };
+    // a quad past the row's end reads the row's first and is zeroed below
+    auto load = [&](int k, Piece &v) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int c = k + c0 + 4 * h;
+            const int at = c < p.in ? c : 0;
+            v.w[h] = ldg4_stream(wr + at);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                v.x[b][h] = ldg4(xr[b] + at);
+        }
+    };
+    d4 acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        acc[b] = d4{0.0, 0.0, 0.0, 0.0};
+    // MFMA k slot kq of step (h, j) holds column c0 + 4h + j
+    auto multiply = [&](int k, const Piece &v) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bool in = k + c0 + 4 * h < p.in;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const double wv = (double)(in ? v.w[h][j] : 0.f);
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        (double)(in ? v.x[b][h][j] : 0.f), wv, acc[b], 0, 0, 0);
+            }
+        }
+    };
+    Piece even, odd;
+    load(0, even);
+    for (int k = 0; k < p.in; k += 2 * kFewStep) {
+        load(k + kFewStep, odd);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(k, even);
+        load(k + 2 * kFewStep, even);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(k + kFewStep, odd);
+    }
+    // acc[b][e]: token 16b + kq + 4e, row r16
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            sums[wave][256 * b + 16 * (kq + 4 * e) + r16] = acc[b][e];
+    __syncthreads();
+    for (int o = tid; o < 256 * NB; o += 64 * kFewWaves) {
+        double s = sums[0][o];
+#pragma unroll
+        for (int w = 1; w < kFewWaves; ++w)
+            s += sums[w][o];
+        const int t = t0 + o / 16, r = r0 + o % 16;
+        if (t < p.n && r < p.out)
+            stg(p.proj + (int64_t)t * p.out + r, (float)s);
+    }
+}
+
 template <int TM, int TN, int TK>
 static hipError_t launch_tile(const BlockParams &p, hipStream_t stream)
 {
@@ -475,9 +571,30 @@ static hipError_t launch_tiles(const BlockParams &p, hipStream_t stream)
     return least->second(p, stream);
 }
 
+// Tokens project_few_kernel takes, by columns that are whole 16-byte quads:
+// from 3 (two tokens: 17.3 us in the row kernel, 19.6 us here) to 64, and to
+// 128 while its 16-row groups are at most one per CU and larger tiles leave
+// the chip idle (2816 x 4096, 80 tokens: 74 us against 97 us in tiles, 128:
+// 86 against 100, 150: 109 against 103).
+constexpr int kFewFrom = 3, kFewTo = 64, kFewToShort = 128;
+
+template <int NB> static void launch_few(const BlockParams &p, hipStream_t stream)
+{
+    const dim3 grid((p.out + 15) / 16, (p.n + 16 * NB - 1) / (16 * NB));
+    project_few_kernel<NB><<<grid, 64 * kFewWaves, 0, stream>>>(p);
+}
+
 hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
 {
-    if (p.n <= kRowTokens) {
+    const int few_to = (p.out + 15) / 16 <= device_cus() ? kFewToShort : kFewTo;
+    if (p.in % 4 == 0 && p.n >= kFewFrom && p.n <= few_to) {
+        if (p.n <= 16)
+            launch_few<1>(p, stream);
+        else if (p.n <= 32 || p.n > 64)
+            launch_few<2>(p, stream); // 128 tokens: 86 us, 95 us with 64 a group
+        else
+            launch_few<4>(p, stream);
+    } else if (p.n <= kRowTokens) {
         const dim3 grid((p.out + 3) / 4);
         if (p.n == 1 && p.in % 4 == 0 && p.in <= kLdsRowFloats)
             project_row_lds_kernel<<<grid, 256, p.in * 4, stream>>>(p, 0);

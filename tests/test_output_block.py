@@ -78,7 +78,7 @@ def run_block(torch, ctx, x, w, scale, res, eps=1e-6, in_place=False):
     return proj.cpu().numpy(), out.cpu().numpy(), err
 
 
-# n = 1, 5, 7, 16: few tokens; 17, 32, 33, 200, 300: f64 MFMA tiles. One token
+# n = 1, 5, 7, 16, 17, 32, 33: few tokens; 200, 300: f64 MFMA tiles. One token
 # with input rows of at most 16384 columns (a multiple of 4) is projected
 # with the input row staged in LDS: rows of 1000 (fewer than 4096 columns),
 # 5000 (4096 and a partial step), 4000 (one 4096-column step taken by some
@@ -112,15 +112,22 @@ def test_output_block_matches_the_oracle(torch, ctx, oracle, case):
     assert same >= 0.999 * n * rows
 
 
-# 17-40 tokens: 32 x 32 tiles, one and two blocks of rows with remainders;
-# 520 x 2816: 64 x 32 or 64 x 64; 530 tokens over 4220 rows: 128 x 64; 1400
-# over 2816: 128 x 128 (the choice follows the device's CU count). Columns
-# below, at and past each K step, and not a multiple of 4.
+# Tiles: 17-40 tokens of 127 or 130 columns take 32 x 32 ones, with
+# remainders of rows and tokens; 520 x 2816: 64 x 32 or 64 x 64; 530 tokens
+# over 4220 rows: 128 x 64; 1400 over 2816: 128 x 128 (the choice follows the
+# device's CU count). Columns below, at and past each K step. The few-token
+# kernel (columns a multiple of 4): 16, 32 and 64 tokens a group and one past
+# each, both ends of its range, output rows of 16 and one past, columns
+# within one wave's 32, one past a 256-column step and past two.
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", [(17, 127, 33), (31, 128, 32), (40, 130, 65), (129, 66, 2816),
+@pytest.mark.parametrize("case", [(17, 127, 33), (31, 126, 32), (40, 130, 65), (129, 68, 2816),
                                   (520, 65, 2816), (700, 63, 2816), (530, 34, 4220),
-                                  (1400, 31, 2816)], ids=lambda c: "x".join(map(str, c)))
-def test_projection_tiles_match_f64_sums(torch, ctx, case):
+                                  (1400, 31, 2816),
+                                  (3, 4, 1), (4, 28, 16), (16, 260, 17), (17, 256, 33),
+                                  (32, 516, 16), (33, 512, 40), (64, 1028, 31), (65, 772, 33),
+                                  (128, 96, 18), (65, 96, 4220), (5, 4096, 2816)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_projection_matches_f64_sums(torch, ctx, case):
     n, cols, rows = case
     g = np.random.default_rng(sum(case))
     x = g.standard_normal((n, cols)).astype(np.float32)
