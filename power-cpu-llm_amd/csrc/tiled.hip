@@ -1,7 +1,8 @@
 // LDS-tiled prefill / canvas attention for gfx950.
 //
 // One workgroup of 8 waves (two per SIMD) owns 128 flat (query, head) rows of
-// one KV head, one 16-row MFMA unit per wave. Q^T (MFMA B operands) and the
+// one KV head, one 16-row MFMA unit per wave; launches that 64-row blocks
+// balance better over the CUs run 4 waves (half_blocks). Q^T (MFMA B operands) and the
 // chunk state O stay in registers. K and V tiles of 32 keys are copied
 // HBM -> LDS by global_load_lds_dwordx4 (no register staging), double
 // buffered. K rows are stored with their 16-byte chunks XOR-swizzled by
@@ -77,11 +78,11 @@ __device__ __forceinline__ bool tile_whole(const Params &p, int row_lo, int row_
     return kmax <= qlo && (p.window == 0 || qhi - kmin < p.window);
 }
 
-// One workgroup per CU (its K/V stages fill the LDS), so at most two waves
-// per SIMD: each wave may hold 256 VGPRs, which the operand double-buffering
-// below uses. W waves per workgroup, one 16-row unit each.
+// One workgroup per CU (its K/V stages fill the LDS), so at most W / 4 waves
+// per SIMD: each wave may hold 256 VGPRs and more, which the operand
+// double-buffering below uses. W waves per workgroup, one 16-row unit each.
 template <int DK, int W, bool CAP>
-__global__ __launch_bounds__(64 * W, 2) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(64 * W, W / 4) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
 void tiled_kernel(Params p, int split, int z0)
 {
     using LD = TiledLds<DK>;
@@ -91,7 +92,7 @@ void tiled_kernel(Params p, int split, int z0)
     constexpr int ROWS = W * kRows;            // rows of the workgroup
     constexpr int NL = LD::spanBlocks;         // span accumulator blocks kept in LDS
     static_assert(NI * W * 256 == kTile * DK, "whole 1 KiB pieces per wave");
-    static_assert(ROWS == kTiledRows, "LDS span blocks sized for the workgroup");
+    static_assert(ROWS <= kTiledRows, "LDS span blocks sized for the workgroup");
     extern __shared__ float lds[];
 
     const int tid = threadIdx.x;
@@ -552,15 +553,59 @@ int tiled_tail_chunks(const Params &p, int nqb, int cus)
     return 1;
 }
 
-template <int DK, bool CAP>
+template <int DK, int W, bool CAP>
 static hipError_t launch_tiled_grid(const Params &p, int split, dim3 grid, hipStream_t stream)
 {
-    const hipError_t e = configure_tiled<DK, kTiledWaves, CAP>();
+    const hipError_t e = configure_tiled<DK, W, CAP>();
     if (e != hipSuccess)
         return e;
-    tiled_kernel<DK, kTiledWaves, CAP>
-        <<<grid, 64 * kTiledWaves, TiledLds<DK>::bytes, stream>>>(p, split, 0);
+    tiled_kernel<DK, W, CAP><<<grid, 64 * W, TiledLds<DK>::bytes, stream>>>(p, split, 0);
     return hipGetLastError();
+}
+
+// Key tiles of the row block [fa, fa + rows), as the kernel bounds them.
+static int64_t block_tiles(const Params &p, int64_t fa, int64_t rows)
+{
+    int64_t k_lo = 0, k_hi = p.nkeys;
+    if (!p.mask && p.causal) {
+        const int64_t fb = std::min<int64_t>(fa + rows, p.nrows) - 1;
+        const int64_t qa = p.first_query + fa / p.group, qz = p.first_query + fb / p.group;
+        k_hi = std::clamp<int64_t>(qz - p.first_key + 1, 0, p.nkeys);
+        if (p.window)
+            k_lo = std::clamp<int64_t>(qa - p.window + 1 - p.first_key, 0, p.nkeys);
+    }
+    return std::max<int64_t>((k_hi + kTile - 1) / kTile - k_lo / kTile, 0);
+}
+
+// Tiles of the CU with the most, over row blocks of `rows` dealt last block
+// first: at least the mean, and at least k + 1 of the k * cus + 1 longest
+// blocks (which the dealing comes close to).
+static int64_t span_tiles(const Params &p, int64_t rows, int64_t cus)
+{
+    const int64_t nqb = (p.nrows + rows - 1) / rows;
+    int64_t total = 0, span = 0;
+    for (int64_t qb = 0; qb < nqb; ++qb)
+        total += block_tiles(p, qb * rows, rows) * p.nkv;
+    for (int64_t k = 0; k * cus < nqb * p.nkv; ++k)
+        span = std::max(span, (k + 1) * block_tiles(p, (nqb - 1 - k * cus / p.nkv) * rows, rows));
+    return std::max(span, (total + cus - 1) / cus);
+}
+
+// Whether 64-row blocks (four waves, one per SIMD) end sooner than 128-row
+// ones. A CU runs a 64-row tile in 0.68 of a 128-row one's time (one wave
+// hides less of its own latency), and several rounds of unequal blocks end
+// up to 15 % past their mean: 0.78 of the tiles must be less. Where one round
+// holds every block the longest decides, and half of it is always less. At
+// head dim 64 two such blocks share a CU, so the mean counts half.
+// Measured, causal prompts of 16 query and 8 KV heads of 256 dims, 128 rows
+// against 64: 1024 tokens 308 -> 209 us, 2048 611 -> 445 us, 2560 765 -> 749
+// us, 1024 over 5000 keys 1491 -> 989 us; 3001 tokens 896 against 1011 us and
+// 4096 1308 against 1686 us keep 128 rows.
+template <int DK> static bool half_blocks(const Params &p)
+{
+    constexpr int kPercent = DK == 64 ? 55 : 78;
+    const int64_t cus = std::max(device_cus(), 1);
+    return kPercent * span_tiles(p, kTiledRows / 2, cus) < 100 * span_tiles(p, kTiledRows, cus);
 }
 
 template <int DK>
@@ -568,9 +613,16 @@ static hipError_t launch_tiled_dk(const Params &p, int split, hipStream_t stream
 {
     const int nqb = (p.nrows + kTiledRows - 1) / kTiledRows;
     const int tail = split ? tiled_tail_chunks(p, nqb, device_cus()) : 0;
+    if (!split && half_blocks<DK>(p)) {
+        constexpr int W = kTiledWaves / 2;
+        const dim3 half((p.nrows + W * kRows - 1) / (W * kRows) * p.nkv);
+        return p.softcap > 0.0f ? launch_tiled_grid<DK, W, true>(p, 0, half, stream)
+                                : launch_tiled_grid<DK, W, false>(p, 0, half, stream);
+    }
     const dim3 grid(nqb * p.nkv, 1, split ? p.nch - tail : 1);
-    hipError_t e = p.softcap > 0.0f ? launch_tiled_grid<DK, true>(p, split, grid, stream)
-                                    : launch_tiled_grid<DK, false>(p, split, grid, stream);
+    hipError_t e = p.softcap > 0.0f
+                       ? launch_tiled_grid<DK, kTiledWaves, true>(p, split, grid, stream)
+                       : launch_tiled_grid<DK, kTiledWaves, false>(p, split, grid, stream);
     if (e != hipSuccess || !tail)
         return e;
     // the tail runs after every other chunk's partial is written: with all

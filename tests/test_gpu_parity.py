@@ -771,6 +771,41 @@ def test_explicit_masks_segments_scale_and_kv_ranges_keep_bits(torch, ctx):
                                                                 6 * group * dim]))
 
 
+# (qheads, kvheads, dim, queries, keys, causal, window): rows one below, at and
+# past 64- and 128-row blocks; one round of blocks (64 rows each), many equal
+# blocks (128 rows each), windows inside key chunks, a padded head dim.
+ROW_BLOCK_CASES = [(2, 1, 256, 31, 300, 1, 0), (2, 1, 256, 32, 300, 1, 0),
+                   (16, 8, 256, 65, 65, 1, 0), (16, 8, 256, 1087, 1087, 1, 500),
+                   (32, 8, 128, 33, 700, 1, 0), (16, 4, 64, 400, 900, 1, 0),
+                   (16, 4, 64, 517, 517, 1, 100), (4, 2, 208, 49, 333, 1, 0),
+                   (16, 8, 256, 2048, 288, 0, 0), (16, 2, 512, 40, 600, 1, 0),
+                   (16, 2, 512, 517, 517, 1, 100), (8, 1, 400, 21, 290, 1, 0)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("softcap", [0.0, 3.0])
+@pytest.mark.parametrize("case", ROW_BLOCK_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_row_blocks_keep_the_split_kernels_bits(torch, ctx, case, softcap):
+    qheads, kvh, dim, nq, nkeys, causal, window = case
+    q = gpu_normals(torch, 0x5EED0811, (nq, qheads, dim)) * (1.0 / 16.0)
+    k = gpu_normals(torch, 0x5EED0812, (nkeys, kvh, dim))
+    v = gpu_normals(torch, 0x5EED0813, (nkeys, kvh, dim))
+    outs = []
+    for kernel in (1, 2):
+        out = torch.full((nq, qheads, dim), float("nan"), device="cuda:0")
+        d = ctx.desc(q=q.data_ptr(), q_stride=qheads * dim, nq=nq, k0=k.data_ptr(),
+                     v0=v.data_ptr(), n0=nkeys, qheads=qheads, kvheads=kvh, dim=dim, kh_first=0,
+                     kh_end=kvh, causal=causal, window=window, first_key=0,
+                     first_query=max(nkeys - nq, 0), softcap=softcap, out=out.data_ptr(),
+                     o_stride=qheads * dim, kernel=kernel)
+        ctx.reserve(ctx.workspace_bytes(d))
+        ctx.launch(d)
+        assert ctx.sync() == 0
+        outs.append(out.cpu().numpy())
+    assert np.array_equal(bits(outs[0]), bits(outs[1]))
+
+
+@pytest.mark.gpu
 def test_long_launch_combines_agree_across_kernels(torch, ctx, oracle):
     """More than 8 spans of 4096 keys: the split kernels' two-level combine
     and the tiled kernel's in-kernel merges give the same bits."""
