@@ -580,7 +580,7 @@ static int64_t block_tiles(const Params &p, int64_t fa, int64_t rows)
 // Tiles of the CU with the most, over row blocks of `rows` dealt last block
 // first: at least the mean, and at least k + 1 of the k * cus + 1 longest
 // blocks (which the dealing comes close to).
-static int64_t span_tiles(const Params &p, int64_t rows, int64_t cus)
+int64_t span_tiles(const Params &p, int64_t rows, int64_t cus)
 {
     const int64_t nqb = (p.nrows + rows - 1) / rows;
     int64_t total = 0, span = 0;

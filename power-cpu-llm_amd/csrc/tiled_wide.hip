@@ -12,7 +12,8 @@
 // tile's online softmax (the same values, bit for bit) and the P.V chain of
 // their own dims.
 //
-// One workgroup of 8 waves owns 64 flat (query, head) rows of one KV head
+// One workgroup of 8 waves owns 64 flat (query, head) rows of one KV head (4
+// waves own 32 rows in launches that balance better so)
 // (4 units; on each SIMD one half-0 and one half-1 wave, so the halves'
 // score phases alternate on the MFMA pipe). K and V tiles of 32 keys (64 KiB
 // each) are copied HBM -> LDS by global_load_lds_dwordx4, single-buffered:
@@ -25,13 +26,13 @@
 // other tiled kernel (tiled.hip); each wave merges its own dims.
 #include "attention_device.hpp"
 
+#include <algorithm>
 #include <atomic>
 
 namespace pcl {
 
 constexpr int kWideDk = 512;
-constexpr int kWideUnits = 4;
-constexpr int kWideWaves = 2 * kWideUnits;
+constexpr int kWideUnits = 4; // of a whole workgroup
 constexpr int kWideRows = kWideUnits * kRows; // 64
 constexpr int kWideTileFloats = kTile * kWideDk;
 // K tile, V tile, half 0's partial score accumulators and half 1's scores
@@ -64,24 +65,25 @@ __device__ __forceinline__ bool wide_tile_whole(const Params &p, int row_lo, int
     return kmax <= qlo && (p.window == 0 || qhi - kmin < p.window);
 }
 
-template <bool CAP>
-__global__ __launch_bounds__(64 * kWideWaves, 2) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void tiled_wide_kernel(Params p, int split, int z0)
+// U units (2 U waves) per workgroup.
+template <int U, bool CAP>
+__device__ __forceinline__ void tiled_wide(const Params &p, int split, int z0)
 {
     constexpr int NU = 8; // score chain steps per half
     constexpr int NQ = 4; // 64-dim output groups per half
-    constexpr int NI = kWideTileFloats / 256 / kWideWaves; // 1 KiB DMA pieces per wave per array
+    constexpr int ROWS = U * kRows;
+    constexpr int NI = kWideTileFloats / 256 / (2 * U); // 1 KiB DMA pieces per wave per array
     extern __shared__ float lds[];
     float *ks = lds;
     float *vs = lds + kWideTileFloats;
     f4 *part = reinterpret_cast<f4 *>(lds + 2 * kWideTileFloats); // [unit][b][lane]
-    f4 *fin = part + kWideUnits * 2 * 64;                          // [unit][b][lane]
+    f4 *fin = part + U * 2 * 64;                          // [unit][b][lane]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wv = tid >> 6;
-    const int unit = wv % kWideUnits;
-    const int half = wv / kWideUnits;
+    const int unit = wv % U;
+    const int half = wv / U;
     const int col = lane & 15;
     const int g = lane >> 4;
     // blocks cycle over the KV heads first; query blocks run last-to-first
@@ -89,7 +91,7 @@ void tiled_wide_kernel(Params p, int split, int z0)
     const int kvl = blockIdx.x % p.nkv;
     const int qb = nqb - 1 - (int)(blockIdx.x / p.nkv);
     const int kh = p.kh_first + kvl;
-    const int fa = qb * kWideRows;
+    const int fa = qb * ROWS;
     const int row = fa + unit * kRows + col;
     const int wrow_lo = fa + unit * kRows;
     const int wrow_hi = min(wrow_lo + kRows, p.nrows) - 1;
@@ -102,7 +104,7 @@ void tiled_wide_kernel(Params p, int split, int z0)
     const RowKeys rk = row_keys(p, row);
     int64_t k_lo = 0, k_hi = p.nkeys;
     if (!p.mask && p.causal) {
-        const int fb = min(fa + kWideRows, p.nrows) - 1;
+        const int fb = min(fa + ROWS, p.nrows) - 1;
         const int64_t qa = p.first_query + fa / p.group;
         const int64_t qz = p.first_query + fb / p.group;
         k_hi = min(max(qz - p.first_key + 1, (int64_t)0), p.nkeys);
@@ -489,12 +491,29 @@ void tiled_wide_kernel(Params p, int split, int z0)
     }
 }
 
+template <bool CAP>
+__global__ __launch_bounds__(128 * kWideUnits, 2) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void tiled_wide_kernel(Params p, int split, int z0)
+{
+    tiled_wide<kWideUnits, CAP>(p, split, z0);
+}
+
+// 32 rows: one wave per SIMD.
+template <bool CAP>
+__global__ __launch_bounds__(64 * kWideUnits, 1) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void tiled_wide_half_kernel(Params p, int split, int z0)
+{
+    tiled_wide<kWideUnits / 2, CAP>(p, split, z0);
+}
+
 constexpr int kWideMaxDevices = 64;
 
 
-template <bool CAP>
+template <int U, bool CAP>
 static hipError_t launch_wide(const Params &p, int split, dim3 grid, hipStream_t stream)
 {
+    static_assert(U == kWideUnits || U == kWideUnits / 2);
+    constexpr auto kernel = U == kWideUnits ? tiled_wide_kernel<CAP> : tiled_wide_half_kernel<CAP>;
     static std::atomic<bool> configured[kWideMaxDevices];
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -503,19 +522,33 @@ static hipError_t launch_wide(const Params &p, int split, dim3 grid, hipStream_t
     if (dev < 0 || dev >= kWideMaxDevices)
         return hipErrorInvalidDevice;
     if (!configured[dev].load(std::memory_order_acquire)) {
-        e = hipFuncSetAttribute((const void *)tiled_wide_kernel<CAP>,
+        e = hipFuncSetAttribute((const void *)kernel,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWideLdsBytes);
         if (e != hipSuccess)
             return e;
         configured[dev].store(true, std::memory_order_release);
     }
-    tiled_wide_kernel<CAP><<<grid, 64 * kWideWaves, kWideLdsBytes, stream>>>(p, split, 0);
+    kernel<<<grid, 128 * U, kWideLdsBytes, stream>>>(p, split, 0);
     return hipGetLastError();
 }
 
 int device_cus();
 int tiled_tail_chunks(const Params &p, int nqb, int cus);
+int64_t span_tiles(const Params &p, int64_t rows, int64_t cus);
 hipError_t launch_fan_chunk(const Params &p, int ci, bool merge_out, hipStream_t stream);
+
+// Whether 32-row blocks (two units, one wave per SIMD) end sooner than
+// 64-row ones: with fewer tiles on the busiest CU, or one round of blocks
+// either way. A SIMD's two waves take turns on the score chains, so half the
+// rows save less here than at head dim 256: a 32-row tile takes 0.9 of a
+// 64-row one's time. Causal prompts of 16 query and 2 KV heads, 64 rows
+// against 32: 128 tokens 53.7 -> 48.2 us, 512 tokens 181 -> 163 us, 768 tokens
+// 266 -> 241 us, 1024 tokens 352 -> 349 us.
+static bool wide_half_blocks(const Params &p)
+{
+    const int64_t cus = std::max(device_cus(), 1);
+    return 95 * span_tiles(p, kWideRows / 2, cus) < 100 * span_tiles(p, kWideRows, cus);
+}
 
 // A split launch whose chunk items leave a small last round runs that
 // round's chunk as fanned (16-row unit, chunk) items (fan_kv.hip), as the
@@ -525,9 +558,15 @@ hipError_t launch_tiled_wide(const Params &p, int split, hipStream_t stream, boo
 {
     const int nqb = (p.nrows + kWideRows - 1) / kWideRows;
     const int tail = split ? tiled_tail_chunks(p, nqb, device_cus()) : 0;
+    if (!split && wide_half_blocks(p)) {
+        constexpr int U = kWideUnits / 2;
+        const dim3 half((p.nrows + U * kRows - 1) / (U * kRows) * p.nkv);
+        return p.softcap > 0.0f ? launch_wide<U, true>(p, 0, half, stream)
+                                : launch_wide<U, false>(p, 0, half, stream);
+    }
     const dim3 grid(nqb * p.nkv, 1, split ? p.nch - tail : 1);
-    hipError_t e = p.softcap > 0.0f ? launch_wide<true>(p, split, grid, stream)
-                                    : launch_wide<false>(p, split, grid, stream);
+    hipError_t e = p.softcap > 0.0f ? launch_wide<kWideUnits, true>(p, split, grid, stream)
+                                    : launch_wide<kWideUnits, false>(p, split, grid, stream);
     if (e != hipSuccess || !tail)
         return e;
     const bool merge_out = p.nspan == 1;

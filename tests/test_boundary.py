@@ -214,7 +214,9 @@ def _resource_remarks(source):
 
 @pytest.mark.parametrize("source,kernel", [
     ("tiled.hip", "_ZN3pcl12tiled_kernelILi256ELi8ELb0EEEvNS_6ParamsEii"),
+    ("tiled.hip", "_ZN3pcl12tiled_kernelILi256ELi4ELb0EEEvNS_6ParamsEii"),
     ("tiled_wide.hip", "_ZN3pcl17tiled_wide_kernelILb0EEEvNS_6ParamsEii"),
+    ("tiled_wide.hip", "_ZN3pcl22tiled_wide_half_kernelILb0EEEvNS_6ParamsEii"),
     ("spread_kv.hip", "_ZN3pcl16spread_kv_kernelILi256ELb1ELb0ELb0ELi2ELb0ELb0EEEvNS_6ParamsE"),
     ("spread_kv.hip", "_ZN3pcl16spread_kv_kernelILi256ELb1ELb0ELb1ELi2ELb0ELb0EEEvNS_6ParamsE"),
     ("spread_kv.hip", "_ZN3pcl16spread_kv_kernelILi256ELb1ELb0ELb1ELi4ELb0ELb0EEEvNS_6ParamsE"),
