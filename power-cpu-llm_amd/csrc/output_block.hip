@@ -4,14 +4,15 @@
 // p9_ref_matvec, src/kernels/portable/reference.rs:36-78).
 //
 // The engine's exact projection sums f64 products of f32 weights and inputs
-// (each product is exact in f64) per output row. Both projection kernels here
-// accumulate in f64 as well, in their own order, so a projected value is the
+// (each product is exact in f64) per output row. Every projection kernel here
+// accumulates in f64 as well, in its own order, so a projected value is the
 // f32 rounding of nearly the same f64 sum: it equals the engine's except when
 // the two f64 sums straddle an f32 rounding boundary, and a sum like
-// 2^24 + 1 - 2^24 stays exact.
+// 2^24 + 1 - 2^24 stays exact. The order depends on the token count only: one
+// for up to 32 tokens (the first three kernels give the same bits), one for
+// more (the tiles of every shape).
 //
-//   project_rows_kernel: one or two tokens (up to 16 where the columns are
-//     not whole 16-byte quads). HBM-bound on the
+//   project_rows_kernel: one or two tokens. HBM-bound on the
 //     weights: one wave per output row streams the row once with 16-byte
 //     loads, 4096 columns in flight at a time, and keeps one f64 accumulator
 //     per token per lane; the tokens' inputs come from L2.
@@ -19,9 +20,9 @@
 //     wide: as project_rows_kernel<1>, with the input row staged once per
 //     workgroup in LDS (requested ahead of the weights) instead of read from
 //     L2 by every wave.
-//   project_few_kernel: 3 to 64 tokens (verification, short prompts; 128 for
-//     few output rows): the waves of a workgroup split the columns of 16
-//     output rows, f64 MFMAs on operands loaded straight from memory.
+//   project_few_kernel: up to 32 tokens (verification, short prompts): the
+//     waves of a workgroup split the columns of 16 output rows, f64 MFMAs on
+//     operands loaded straight from memory.
 //   project_tiles_kernel: more tokens (prompt). MFMA-bound: output
 //     tiles of 128 x 128 down to 32 x 32, K steps double-buffered in LDS as
 //     f32, the products on v_mfma_f64_16x16x4f64 after converting the
@@ -38,6 +39,7 @@
 #include <atomic>
 #include <cstdio>
 #include <iterator>
+#include <type_traits>
 #include <utility>
 
 namespace pcl {
@@ -60,24 +62,15 @@ struct BlockParams {
     int *err;
 };
 
-// Largest token count of the row kernel (columns that are not whole 16-byte
-// quads; else two tokens): 16 tokens run 55 us there and 66 us in tiles (2816
-// x 4096), 17-32 tokens took it two passes (24 tokens 108 us, in tiles 67 us).
-constexpr int kRowTokens = 16;
-
-// One wave per output row; tokens [t0, t0 + min(NT, n - t0)) per launch
-// pass. Instantiated for NT = 1, 2, 4, 8 and 16: a one-token decode then
-// carries no per-token tests for 15 absent tokens in its inner loop (that
-// made the 2816 x 4096 projection 15 us against 9 us). Every token's f64 sum
-// runs in the same order in every instantiation.
+// One wave per output row, NT = n tokens. Every token's f64 sum runs in the
+// same order in every instantiation.
 template <int NT>
-__global__ __launch_bounds__(256) void project_rows_kernel(BlockParams p, int t0)
+__global__ __launch_bounds__(256) void project_rows_kernel(BlockParams p)
 {
     const int lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= p.out)
         return;
-    const int nt = p.n - t0 < NT ? p.n - t0 : NT;
     const float *wr = p.w + (int64_t)r * p.in;
     double acc[NT];
 #pragma unroll
@@ -96,12 +89,10 @@ __global__ __launch_bounds__(256) void project_rows_kernel(BlockParams p, int t0
         for (int k = 0; k < 16; ++k) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                if (t < nt) {
-                    const f4 xv = ldg4(p.x + (int64_t)(t0 + t) * p.in + 4 * (v + 64 * k));
+                const f4 xv = ldg4(p.x + (int64_t)t * p.in + 4 * (v + 64 * k));
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        acc[t] = __builtin_fma((double)wv[k][e], (double)xv[e], acc[t]);
-                }
+                for (int e = 0; e < 4; ++e)
+                    acc[t] = __builtin_fma((double)wv[k][e], (double)xv[e], acc[t]);
             }
         }
     }
@@ -109,12 +100,10 @@ __global__ __launch_bounds__(256) void project_rows_kernel(BlockParams p, int t0
         const f4 wv = ldg4_stream(wr + 4 * v);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            if (t < nt) {
-                const f4 xv = ldg4(p.x + (int64_t)(t0 + t) * p.in + 4 * v);
+            const f4 xv = ldg4(p.x + (int64_t)t * p.in + 4 * v);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    acc[t] = __builtin_fma((double)wv[e], (double)xv[e], acc[t]);
-            }
+            for (int e = 0; e < 4; ++e)
+                acc[t] = __builtin_fma((double)wv[e], (double)xv[e], acc[t]);
         }
     }
     // columns past the last whole 16-byte step
@@ -122,25 +111,22 @@ __global__ __launch_bounds__(256) void project_rows_kernel(BlockParams p, int t0
         const double wc = (double)ldg(wr + c);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-            if (t < nt)
-                acc[t] = __builtin_fma(wc, (double)ldg(p.x + (int64_t)(t0 + t) * p.in + c), acc[t]);
+            acc[t] = __builtin_fma(wc, (double)ldg(p.x + (int64_t)t * p.in + c), acc[t]);
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-        if (t < nt) {
-            double s = acc[t];
+        double s = acc[t];
 #pragma unroll
-            for (int o = 32; o >= 1; o >>= 1)
-                s += __shfl_xor(s, o);
-            acc[t] = s;
-        }
+        for (int o = 32; o >= 1; o >>= 1)
+            s += __shfl_xor(s, o);
+        acc[t] = s;
     }
-    if (lane < nt) {
+    if (lane < NT) {
         double mine = 0.0;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
             mine = lane == t ? acc[t] : mine;
-        stg(p.proj + (int64_t)(t0 + lane) * p.out + r, (float)mine);
+        stg(p.proj + (int64_t)lane * p.out + r, (float)mine);
     }
 }
 
@@ -350,12 +336,12 @@ __global__ __launch_bounds__(256) void post_norm_kernel(BlockParams p)
 // The largest input row project_row_lds_kernel stages (64 KiB of LDS).
 constexpr int kLdsRowFloats = 16384;
 
-// One token t0 (p.in % 4 == 0, p.in <= kLdsRowFloats), one wave per output
+// One token (p.in % 4 == 0, p.in <= kLdsRowFloats), one wave per output
 // row as in project_rows_kernel<1> (the same f64 sums in the same order):
 // the workgroup stages the input row in LDS once, its first 4096 columns
 // requested before the rows' first weights so that the LDS stores wait only
 // for them.
-__global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p, int t0)
+__global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p)
 {
     extern __shared__ f4 xs[];
     const int lane = threadIdx.x & 63;
@@ -364,7 +350,7 @@ __global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p, int
     const bool live = r < p.out;
     // a wave past the last row streams row 0 (in bounds; unused)
     const float *wr = p.w + (int64_t)(live ? r : 0) * p.in;
-    const float *xr = p.x + (int64_t)t0 * p.in;
+    const float *xr = p.x;
     f4 wv[16];
     int v = lane;
     if (vecs >= 1024) {
@@ -419,32 +405,60 @@ __global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p, int
     for (int o = 32; o >= 1; o >>= 1)
         acc += __shfl_xor(acc, o);
     if (lane == 0)
-        stg(p.proj + (int64_t)t0 * p.out + r, (float)acc);
+        stg(p.proj + r, (float)acc);
+}
+
+// The 4 x 4 transpose of four registers over a wave's four 16-lane groups:
+// lane group g's element i becomes lane group i's element g.
+__device__ __forceinline__ f4 transpose_groups(f4 v)
+{
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[2]),
+                                                    false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[1]), __float_as_uint(v[3]),
+                                                    false, false);
+    const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    return f4{__uint_as_float(lo[0]), __uint_as_float(lo[1]), __uint_as_float(hi[0]),
+              __uint_as_float(hi[1])};
 }
 
 // 16 output rows x 16 NB tokens per workgroup, its eight waves splitting the
-// columns: 32-column pieces go round the waves (256 columns, 1 KiB of a row,
-// per step). Bound by the weights' stream and its round trips: a wave loads
-// MFMA operands straight from memory (every weight is used by one wave only,
-// so LDS would add a pass), one piece requested ahead of the piece being
-// multiplied (two or four ahead were slower, 16 tokens 24.2 against 24.5 and
-// 27.3 us). The waves' f64 sums meet in LDS and are added in wave order.
-// p.in % 4 == 0. Projection of 2816 x 4096 with its post-norm, one wave per
-// row (in tiles past 16 tokens) against this: 4 tokens 22.9 -> 19.1 us, 16
-// tokens 53 -> 24.2 us, 32 tokens 66 -> 31.9 us, 64 tokens 69 -> 50.9 us.
+// columns. A wave loads MFMA operands straight from memory (every weight is
+// used by one wave only, so LDS would add a pass), the next 256 columns'
+// requested ahead of the ones being multiplied.
+//
+// Every output is the sum that project_rows_kernel forms, bit for bit, so a
+// token's row does not depend on how many tokens come with it: that kernel's
+// lane l sums the 16-byte quads l, l + 64, ... of a row, and here each l has
+// an accumulator of its own, wave w those of lanes 4w to 4w + 3 and 32 + 4w to
+// 35 + 4w. The f64 MFMA adds its four k slots as an ascending chain of fmas;
+// transposing the quads over the lane groups makes the slots the quad's
+// columns. The lane sums meet as in the shuffles there: over lanes 32 in the
+// wave, 16, 8 and 4 with other waves through LDS, 2 and 1 in the wave.
+//
+// Bound by the weights' stream and its round trips, at 32 tokens also by the
+// MFMAs of the CUs that have a group of rows (13.7 us of the 35 at 4096
+// columns, at the fp64 peak). 2816 x 4096 with its post-norm, one wave per row against
+// this: 5 tokens 25.5 -> 20.2 us, 16 tokens 52 -> 25.3 us, 32 tokens 117 ->
+// 35.2 us. Eight accumulators a token block of the wave, the transposes and
+// the exchange cost 0.6 to 3.5 us of it against sums in whatever order is
+// nearest (16 tokens 24.2, 32 tokens 31.8 us).
 constexpr int kFewWaves = 8;
-constexpr int kFewStep = 32 * kFewWaves; // columns per piece of all waves
+constexpr int kFewStep = 256; // columns per step: one quad of every lane sum
 
 template <int NB>
 __global__ __launch_bounds__(64 * kFewWaves, 2) void project_few_kernel(BlockParams p)
 {
-    __shared__ double sums[kFewWaves][NB * 256];
+    static_assert(NB == 1 || NB == 2, "half of the waves gather a token block's sums");
+    // partner sums of the waves that gather: [wave][accumulator][element][lane]
+    __shared__ double sums[4 * NB][4][4][64];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
     const int r0 = blockIdx.x * 16, t0 = blockIdx.y * 16 * NB;
-    const int c0 = 32 * wave + 8 * kq; // this lane's first column of piece 0
+    const int c0 = 16 * wave + 4 * kq; // this lane's first column
+    const int whole = p.in & ~3;       // columns in whole quads
     // rows and tokens past the last repeat it (not written)
     const float *wr = p.w + (int64_t)min(r0 + r16, p.out - 1) * p.in;
     const float *xr[NB];
@@ -455,62 +469,138 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void project_few_kernel(BlockPar
     struct Piece {
         f4 w[2], x[NB][2];
     };
-    // a quad past the row's end reads the row's first and is zeroed below
+    // a quad past the last whole one reads the row's first and is zeroed below
     auto load = [&](int k, Piece &v) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int c = k + c0 + 4 * h;
-            const int at = c < p.in ? c : 0;
+            const int c = k + c0 + 128 * h;
+            const int at = c < whole ? c : 0;
             v.w[h] = ldg4_stream(wr + at);
 #pragma unroll
             for (int b = 0; b < NB; ++b)
                 v.x[b][h] = ldg4(xr[b] + at);
         }
     };
-    d4 acc[NB];
+    // acc[b][h][i]: the sums of lane 32 h + 4 wave + i of project_rows_kernel
+    d4 acc[NB][2][4];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
-        acc[b] = d4{0.0, 0.0, 0.0, 0.0};
-    // MFMA k slot kq of step (h, j) holds column c0 + 4h + j
-    auto multiply = [&](int k, const Piece &v) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[b][h][i] = d4{0.0, 0.0, 0.0, 0.0};
+    // masked: the step may hold quads past the last whole one
+    auto multiply = [&](int k, const Piece &v, auto masked) {
+        const f4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const bool in = k + c0 + 4 * h < p.in;
+            const bool in = !masked || k + c0 + 128 * h < whole;
+            const f4 w = transpose_groups(in ? v.w[h] : zero);
+            f4 x[NB];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const double wv = (double)(in ? v.w[h][j] : 0.f);
+            for (int b = 0; b < NB; ++b)
+                x[b] = transpose_groups(in ? v.x[b][h] : zero);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
-                    acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        (double)(in ? v.x[b][h][j] : 0.f), wv, acc[b], 0, 0, 0);
-            }
+                    acc[b][h][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        (double)x[b][i], (double)w[i], acc[b][h][i], 0, 0, 0);
         }
     };
-    Piece even, odd;
-    load(0, even);
-    for (int k = 0; k < p.in; k += 2 * kFewStep) {
-        load(k + kFewStep, odd);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(k, even);
-        load(k + 2 * kFewStep, even);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(k + kFewStep, odd);
+    if (whole > 0) {
+        Piece even, odd;
+        load(0, even);
+        int k = 0;
+        for (; k + 2 * kFewStep <= whole; k += 2 * kFewStep) {
+            load(k + kFewStep, odd);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(k, even, std::false_type{});
+            load(k + 2 * kFewStep, even);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(k + kFewStep, odd, std::false_type{});
+        }
+        if (k < whole) {
+            load(k + kFewStep, odd);
+            multiply(k, even, std::true_type{});
+            multiply(k + kFewStep, odd, std::true_type{});
+        }
     }
-    // acc[b][e]: token 16b + kq + 4e, row r16
+    // columns past the last whole quad belong to lanes 0, 1 and 2
+    if (wave == 0) {
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+        for (int l = 0; l < 3; ++l) {
+            const int c = whole + l;
+            if (c < p.in) {
+                const double w = kq == 0 ? (double)ldg(wr + c) : 0.0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            sums[wave][256 * b + 16 * (kq + 4 * e) + r16] = acc[b][e];
+                for (int b = 0; b < NB; ++b)
+                    acc[b][0][l] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        kq == 0 ? (double)ldg(xr[b] + c) : 0.0, w, acc[b][0][l], 0, 0, 0);
+            }
+        }
+    }
+
+    // Waves 0-3 gather token block 0, waves 4-7 block 1.
+    auto put = [&](int slot, const d4 (&v)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sums[slot][i][e][lane] = v[i][e];
+    };
+    d4 s[4];
+    auto add = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s[i][e] += sums[slot][i][e][lane];
+    };
+    auto halves = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            s[i] = acc[b][0][i] + acc[b][1][i];
+    };
+    const bool upper = wave >= 4;
+    const bool gathers = NB == 2 || !upper;
+    const int mine = upper ? NB - 1 : 0;
+    if (upper) {
+        halves(0);
+        put(wave ^ 4, s);
+        if (NB == 2)
+            halves(NB - 1);
+    } else {
+        if (NB == 2) {
+            halves(NB - 1);
+            put(wave ^ 4, s);
+        }
+        halves(0);
+    }
     __syncthreads();
-    for (int o = tid; o < 256 * NB; o += 64 * kFewWaves) {
-        double s = sums[0][o];
+    if (gathers) {
+        add(wave);
+        if (wave & 2)
+            put(wave, s); // only this wave's own lanes have read the slot
+    }
+    __syncthreads();
+    if (gathers && !(wave & 2)) {
+        add(wave ^ 2);
+        if (wave & 1)
+            put(wave, s);
+    }
+    __syncthreads();
+    if (!gathers || (wave & 3))
+        return;
+    add(wave ^ 1);
+    // element e: token 16 mine + kq + 4e, row r16
+    const d4 sum = (s[0] + s[2]) + (s[1] + s[3]);
 #pragma unroll
-        for (int w = 1; w < kFewWaves; ++w)
-            s += sums[w][o];
-        const int t = t0 + o / 16, r = r0 + o % 16;
+    for (int e = 0; e < 4; ++e) {
+        const int t = t0 + 16 * mine + kq + 4 * e, r = r0 + r16;
         if (t < p.n && r < p.out)
-            stg(p.proj + (int64_t)t * p.out + r, (float)s);
+            stg(p.proj + (int64_t)t * p.out + r, (float)sum[e]);
     }
 }
 
@@ -543,8 +633,8 @@ static hipError_t launch_tile(const BlockParams &p, hipStream_t stream)
 // large tiles, while small ones reach a lower MFMA rate. The constants are
 // measured (4096 columns, one MI355X, us): a tile's share of its CU's time,
 // and the fill and drain of a launch. Projection of 2816 rows, 128 x 128
-// alone against the chosen tile: 33 tokens 568 -> 67 us, 256 tokens 578 ->
-// 152 us, 1000 tokens 590 -> 468 us, 2000 tokens 1080 -> 868 us; 4096 tokens
+// alone against the chosen tile: 33 tokens 567 -> 68 us, 256 tokens 580 ->
+// 159 us, 1000 tokens 593 -> 469 us, 2000 tokens 1078 -> 866 us; 4096 tokens
 // keep 128 x 128 (1.61 ms, 0.74 of the fp64 MFMA peak).
 static hipError_t launch_tiles(const BlockParams &p, hipStream_t stream)
 {
@@ -571,43 +661,29 @@ static hipError_t launch_tiles(const BlockParams &p, hipStream_t stream)
     return least->second(p, stream);
 }
 
-// Tokens project_few_kernel takes, by columns that are whole 16-byte quads:
-// from 3 (two tokens: 17.3 us in the row kernel, 19.6 us here) to 64, and to
-// 128 while its 16-row groups are at most one per CU and larger tiles leave
-// the chip idle (2816 x 4096, 80 tokens: 74 us against 97 us in tiles, 128:
-// 86 against 100, 150: 109 against 103).
-constexpr int kFewFrom = 3, kFewTo = 64, kFewToShort = 128;
-
-template <int NB> static void launch_few(const BlockParams &p, hipStream_t stream)
-{
-    const dim3 grid((p.out + 15) / 16, (p.n + 16 * NB - 1) / (16 * NB));
-    project_few_kernel<NB><<<grid, 64 * kFewWaves, 0, stream>>>(p);
-}
+// Tokens project_few_kernel takes: from 3, up to the 32 that two 16-token
+// blocks of a workgroup hold. Past 16 tokens each workgroup takes both (the
+// weights are read once) unless single blocks fit one round of the CUs
+// (2048 x 2048, 32 tokens: 15.5 us in single blocks, 19.0 us in pairs; 2816 x
+// 4096: 42.7 us against 35.2 us).
+constexpr int kFewFrom = 3, kFewTo = 32;
 
 hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
 {
-    const int few_to = (p.out + 15) / 16 <= device_cus() ? kFewToShort : kFewTo;
-    if (p.in % 4 == 0 && p.n >= kFewFrom && p.n <= few_to) {
-        if (p.n <= 16)
-            launch_few<1>(p, stream);
-        else if (p.n <= 32 || p.n > 64)
-            launch_few<2>(p, stream); // 128 tokens: 86 us, 95 us with 64 a group
-        else
-            launch_few<4>(p, stream);
-    } else if (p.n <= kRowTokens) {
+    if (p.n < kFewFrom) {
         const dim3 grid((p.out + 3) / 4);
         if (p.n == 1 && p.in % 4 == 0 && p.in <= kLdsRowFloats)
-            project_row_lds_kernel<<<grid, 256, p.in * 4, stream>>>(p, 0);
+            project_row_lds_kernel<<<grid, 256, p.in * 4, stream>>>(p);
         else if (p.n == 1)
-            project_rows_kernel<1><<<grid, 256, 0, stream>>>(p, 0);
-        else if (p.n == 2)
-            project_rows_kernel<2><<<grid, 256, 0, stream>>>(p, 0);
-        else if (p.n <= 4)
-            project_rows_kernel<4><<<grid, 256, 0, stream>>>(p, 0);
-        else if (p.n <= 8)
-            project_rows_kernel<8><<<grid, 256, 0, stream>>>(p, 0);
+            project_rows_kernel<1><<<grid, 256, 0, stream>>>(p);
         else
-            project_rows_kernel<16><<<grid, 256, 0, stream>>>(p, 0);
+            project_rows_kernel<2><<<grid, 256, 0, stream>>>(p);
+    } else if (p.n <= kFewTo) {
+        const int rows = (p.out + 15) / 16, blocks = (p.n + 15) / 16;
+        if (blocks == 1 || blocks * rows <= device_cus())
+            project_few_kernel<1><<<dim3(rows, blocks), 64 * kFewWaves, 0, stream>>>(p);
+        else
+            project_few_kernel<2><<<rows, 64 * kFewWaves, 0, stream>>>(p);
     } else {
         const hipError_t e = launch_tiles(p, stream);
         if (e != hipSuccess)

@@ -164,6 +164,45 @@ def test_one_token_projection_equals_the_multi_token_one_bitwise(torch, ctx, col
     assert np.array_equal(out1[0].view(np.uint32), out2[1].view(np.uint32))
 
 
+# A token's projection is the same f64 sum, in one order, in every launch of up
+# to 32 tokens, and in one order in every larger one. Columns: below one quad,
+# whole 256-column steps and one quad past, remainders of one to three columns,
+# more than one 4096-column step, a lone 256-column step; output rows of 16 and
+# one past, enough of them for two 16-token blocks a workgroup. Past 32 tokens:
+# remainders of tokens, rows and columns in tiles of several shapes, each over
+# more than two K steps. The terms of a row cancel in pairs but for a few small
+# ones, so that f64 sums in another order differ in their f32 bits.
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [(3, 4096, 300), (2, 1001, 33), (4, 1000, 300), (5, 8193, 16),
+                                  (8, 4098, 17), (16, 260, 64), (16, 1, 1), (17, 4096, 130),
+                                  (31, 1003, 48), (32, 512, 4200), (17, 259, 2816), (32, 3, 4200),
+                                  (34, 4097, 33), (64, 1028, 300), (128, 196, 65),
+                                  (200, 1000, 2816), (520, 515, 2816), (700, 261, 2816),
+                                  (1400, 133, 2816), (2100, 130, 2816)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_a_tokens_projection_does_not_depend_on_the_token_count(torch, ctx, case):
+    n, cols, rows = case
+    g = np.random.default_rng(sum(case))
+    h = cols // 2
+    x = (g.standard_normal((n, cols)) * 2.0 ** g.integers(-12, 13, (n, cols))).astype(np.float32)
+    w = (g.standard_normal((rows, cols)) * 2.0 ** g.integers(-12, 13, cols)).astype(np.float32)
+    order = g.permutation(cols)
+    x[:, order[h:2 * h]] = x[:, order[:h]]
+    w[:, order[h:2 * h]] = -w[:, order[:h]]
+    w[:, order[:h // 8]] += np.float32(1e-6)
+    scale = (1 + 0.1 * g.standard_normal(rows)).astype(np.float32)
+    res = g.standard_normal((n, rows)).astype(np.float32)
+    proj, out, err = run_block(torch, ctx, x, w, scale, res)
+    assert err == 0
+    few = 1 if n <= 32 else 33
+    for t in sorted({0, (n - few) // 2, n - few}):
+        rows_t = slice(t, t + few)
+        proj1, out1, err1 = run_block(torch, ctx, x[rows_t], w, scale, res[rows_t])
+        assert err1 == 0
+        assert np.array_equal(proj[rows_t].view(np.uint32), proj1.view(np.uint32))
+        assert np.array_equal(out[rows_t].view(np.uint32), out1.view(np.uint32))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 40])
 def test_output_block_keeps_f64_cancellation_and_runs_in_place(torch, ctx, oracle, n):
