@@ -12,7 +12,7 @@
 // for up to 32 tokens (the first three kernels give the same bits), one for
 // more (the tiles of every shape).
 //
-//   project_rows_kernel: one or two tokens. HBM-bound on the
+//   project_rows_kernel: up to five tokens. HBM-bound on the
 //     weights: one wave per output row streams the row once with 16-byte
 //     loads, 4096 columns in flight at a time, and keeps one f64 accumulator
 //     per token per lane; the tokens' inputs come from L2.
@@ -62,8 +62,9 @@ struct BlockParams {
     int *err;
 };
 
-// One wave per output row, NT = n tokens. Every token's f64 sum runs in the
-// same order in every instantiation.
+// One wave per output row, NT = n tokens (a kernel for each count: tests for
+// absent tokens in the inner loop cost 1 to 5 us at 2 to 4 tokens). Every
+// token's f64 sum runs in the same order in every instantiation.
 template <int NT>
 __global__ __launch_bounds__(256) void project_rows_kernel(BlockParams p)
 {
@@ -439,7 +440,7 @@ __device__ __forceinline__ f4 transpose_groups(f4 v)
 // Bound by the weights' stream and its round trips, at 32 tokens also by the
 // MFMAs of the CUs that have a group of rows (13.7 us of the 35 at 4096
 // columns, at the fp64 peak). 2816 x 4096 with its post-norm, one wave per row against
-// this: 5 tokens 25.5 -> 20.2 us, 16 tokens 52 -> 25.3 us, 32 tokens 117 ->
+// this: 8 tokens 33.2 -> 21.4 us, 16 tokens 52 -> 25.3 us, 32 tokens 117 ->
 // 35.2 us. Eight accumulators a token block of the wave, the transposes and
 // the exchange cost 0.6 to 3.5 us of it against sums in whatever order is
 // nearest (16 tokens 24.2, 32 tokens 31.8 us).
@@ -661,12 +662,15 @@ static hipError_t launch_tiles(const BlockParams &p, hipStream_t stream)
     return least->second(p, stream);
 }
 
-// Tokens project_few_kernel takes: from 3, up to the 32 that two 16-token
-// blocks of a workgroup hold. Past 16 tokens each workgroup takes both (the
-// weights are read once) unless single blocks fit one round of the CUs
-// (2048 x 2048, 32 tokens: 15.5 us in single blocks, 19.0 us in pairs; 2816 x
-// 4096: 42.7 us against 35.2 us).
-constexpr int kFewFrom = 3, kFewTo = 32;
+// Tokens project_few_kernel takes: from 6 (one wave per row spreads over more
+// CUs; 3 tokens 8192 -> 5376 rows of weights 59.7 us there and 71.6 us here,
+// 16384 -> 1024 34.0 and 55.8 us, 4096 -> 2816 17.7 and 19.5 us; 5 tokens 4096
+// -> 2816 19.8 and 20.0 us; 6 tokens 25.8 and 20.4 us) up to the 32 that two
+// 16-token blocks of a workgroup hold. Past 16 tokens each workgroup takes
+// both (the weights are read once) unless single blocks fit one round of the
+// CUs (2048 x 2048, 32 tokens: 15.5 us in single blocks, 19.0 us in pairs;
+// 2816 x 4096: 42.7 us against 35.2 us).
+constexpr int kFewFrom = 6, kFewTo = 32;
 
 hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
 {
@@ -676,8 +680,14 @@ hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
             project_row_lds_kernel<<<grid, 256, p.in * 4, stream>>>(p);
         else if (p.n == 1)
             project_rows_kernel<1><<<grid, 256, 0, stream>>>(p);
-        else
+        else if (p.n == 2)
             project_rows_kernel<2><<<grid, 256, 0, stream>>>(p);
+        else if (p.n == 3)
+            project_rows_kernel<3><<<grid, 256, 0, stream>>>(p);
+        else if (p.n == 4)
+            project_rows_kernel<4><<<grid, 256, 0, stream>>>(p);
+        else
+            project_rows_kernel<5><<<grid, 256, 0, stream>>>(p);
     } else if (p.n <= kFewTo) {
         const int rows = (p.out + 15) / 16, blocks = (p.n + 15) / 16;
         if (blocks == 1 || blocks * rows <= device_cus())
