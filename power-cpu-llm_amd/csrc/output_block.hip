@@ -165,36 +165,41 @@ __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
     const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
 
     // global -> registers -> LDS; the next step's loads are in flight during
-    // this step's MFMAs
+    // this step's MFMAs. Rows past the last repeat it (not written), columns
+    // past the last are zero: a branch around each load of a whole step cost
+    // 6 to 16 % (64 tokens of 4096 columns 69 -> 60 us, 2000 tokens 866 -> 791).
     f4 ra[kLoadA], rb[kLoadB];
     auto load = [&](int k0) {
+        if (k0 + TK <= p.in) { // all loads go out together
+#pragma unroll
+            for (int i = 0; i < kLoadA; ++i) {
+                const int idx = tid + 256 * i;
+                ra[i] = ldg4(p.x + (int64_t)min(m0 + idx / kQuads, p.n - 1) * p.in + k0 +
+                             4 * (idx % kQuads));
+            }
+#pragma unroll
+            for (int i = 0; i < kLoadB; ++i) {
+                const int idx = tid + 256 * i;
+                rb[i] = ldg4_stream(p.w + (int64_t)min(n0 + idx / kQuads, p.out - 1) * p.in + k0 +
+                                    4 * (idx % kQuads));
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < kLoadA; ++i) {
             const int idx = tid + 256 * i;
-            const int row = idx / kQuads, k = k0 + 4 * (idx % kQuads);
-            ra[i] = f4{0.f, 0.f, 0.f, 0.f};
-            if (m0 + row < p.n) {
-                const float *src = p.x + (int64_t)(m0 + row) * p.in;
-                if (k + 3 < p.in)
-                    ra[i] = ldg4(src + k);
-                else
-                    for (int e = 0; e < 4; ++e)
-                        ra[i][e] = k + e < p.in ? ldg(src + k + e) : 0.f;
-            }
+            const int k = k0 + 4 * (idx % kQuads);
+            const float *src = p.x + (int64_t)min(m0 + idx / kQuads, p.n - 1) * p.in + k;
+            for (int e = 0; e < 4; ++e)
+                ra[i][e] = k + e < p.in ? ldg(src + e) : 0.f;
         }
 #pragma unroll
         for (int i = 0; i < kLoadB; ++i) {
             const int idx = tid + 256 * i;
-            const int row = idx / kQuads, k = k0 + 4 * (idx % kQuads);
-            rb[i] = f4{0.f, 0.f, 0.f, 0.f};
-            if (n0 + row < p.out) {
-                const float *src = p.w + (int64_t)(n0 + row) * p.in;
-                if (k + 3 < p.in)
-                    rb[i] = ldg4_stream(src + k);
-                else
-                    for (int e = 0; e < 4; ++e)
-                        rb[i][e] = k + e < p.in ? ldg(src + k + e) : 0.f;
-            }
+            const int k = k0 + 4 * (idx % kQuads);
+            const float *src = p.w + (int64_t)min(n0 + idx / kQuads, p.out - 1) * p.in + k;
+            for (int e = 0; e < 4; ++e)
+                rb[i][e] = k + e < p.in ? ldg(src + e) : 0.f;
         }
     };
     auto store = [&](int buf) {
@@ -634,9 +639,10 @@ static hipError_t launch_tile(const BlockParams &p, hipStream_t stream)
 // large tiles, while small ones reach a lower MFMA rate. The constants are
 // measured (4096 columns, one MI355X, us): a tile's share of its CU's time,
 // and the fill and drain of a launch. Projection of 2816 rows, 128 x 128
-// alone against the chosen tile: 33 tokens 567 -> 68 us, 256 tokens 580 ->
-// 159 us, 1000 tokens 593 -> 469 us, 2000 tokens 1078 -> 866 us; 4096 tokens
-// keep 128 x 128 (1.61 ms, 0.74 of the fp64 MFMA peak).
+// alone (its loads branching over rows and columns) against the chosen tile:
+// 33 tokens 568 -> 60 us, 256 tokens 584 -> 142 us, 1000 tokens 592 -> 425 us,
+// 2000 tokens 1081 -> 791 us; 4096 tokens keep 128 x 128 (1.63 -> 1.55 ms, 0.78
+// of the fp64 MFMA peak).
 static hipError_t launch_tiles(const BlockParams &p, hipStream_t stream)
 {
     const int64_t cus = std::max(device_cus(), 1);
