@@ -85,6 +85,7 @@ EXPORTS = (
     "pcl_kv_cache_append_transformed",
     "pcl_kv_cache_attend_token",
     "pcl_attention_output",
+    "pcl_debug_projection_form",
     "pcl_version",
 )
 
@@ -217,7 +218,8 @@ def load():
             ("pcl_kv_cache_attend_token", ctypes.c_int,
              [vp, vp, vp, vp, vp, ctypes.c_float, ctypes.c_int, vp, vp, pend]),
             ("pcl_attention_output", ctypes.c_int,
-             [vp, vp, i64, i64, vp, i64, vp, ctypes.c_float, vp, vp, vp])):
+             [vp, vp, i64, i64, vp, i64, vp, ctypes.c_float, vp, vp, vp]),
+            ("pcl_debug_projection_form", ctypes.c_int, [i64, i64, i64, ctypes.c_int])):
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args

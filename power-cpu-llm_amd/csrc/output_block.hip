@@ -40,7 +40,6 @@
 #include <cstdio>
 #include <iterator>
 #include <type_traits>
-#include <utility>
 
 namespace pcl {
 
@@ -633,39 +632,47 @@ static hipError_t launch_tile(const BlockParams &p, hipStream_t stream)
     return hipGetLastError();
 }
 
-// The tile with the least time by tiles per CU: the CU with the most tiles
-// sets it, so 352 tiles of 128 x 128 (2000 tokens, 2816 rows) cost two
-// rounds for 1.4 rounds of work, and a few tokens leave most CUs idle under
-// large tiles, while small ones reach a lower MFMA rate. The constants are
-// measured (4096 columns, one MI355X, us): a tile's share of its CU's time,
-// and the fill and drain of a launch. Projection of 2816 rows, 128 x 128
-// alone (its loads branching over rows and columns) against the chosen tile:
-// 33 tokens 568 -> 60 us, 256 tokens 584 -> 142 us, 1000 tokens 592 -> 425 us,
-// 2000 tokens 1081 -> 791 us; 4096 tokens keep 128 x 128 (1.63 -> 1.55 ms, 0.78
-// of the fp64 MFMA peak).
-static hipError_t launch_tiles(const BlockParams &p, hipStream_t stream)
+// The tile shapes and their time by the busiest CU's rounds of tiles: every
+// K step of a shape costs `fill` once and `round` for each tile the CU works
+// (10 ns units, fitted over 33 to 4096 tokens, 64 to 16384 columns and 16 to
+// 11264 output rows on one MI355X; columns are whole K steps, so a row of 96
+// pays for 128 in the smallest tile).
+struct Tile {
+    int m, n, k;
+    int fill, round;
+    hipError_t (*launch)(const BlockParams &, hipStream_t);
+};
+constexpr Tile kTiles[] = {
+    {128, 128, 32, 49, 369, launch_tile<128, 128, 32>},
+    {128, 64, 32, 30, 198, launch_tile<128, 64, 32>},
+    {64, 64, 64, 37, 203, launch_tile<64, 64, 64>},
+    {64, 32, 64, 42, 104, launch_tile<64, 32, 64>},
+    {32, 32, 128, 30, 126, launch_tile<32, 32, 128>},
+};
+
+// The tile with the least time: 352 tiles of 128 x 128 (2000 tokens, 2816
+// rows) cost two rounds for 1.4 rounds of work, and a few tokens leave most
+// CUs idle under large tiles, while small ones reach a lower MFMA rate. Of 224
+// sizes timed in every shape the choice is 0.6 % from the best on average.
+// Projection of 2816 rows of 4096 columns, 128 x 128 alone (its loads
+// branching over rows and columns) against the chosen tile: 33 tokens 568 ->
+// 60 us, 256 tokens 581 -> 139 us, 1000 tokens 589 -> 421 us, 2000 tokens 1076
+// -> 783 us, 4096 tokens 1.62 -> 1.49 ms (0.81 of the fp64 MFMA peak); 2000
+// tokens of 96 columns 44 -> 38 us (49 us by a rule without the column count).
+const Tile &choose_tile(int64_t n, int64_t in, int64_t out, int64_t cus)
 {
-    const int64_t cus = std::max(device_cus(), 1);
-    auto cost = [&](int tm, int tn, int fixed, int per_tile) {
-        const int64_t tiles = (int64_t)((p.out + tn - 1) / tn) * ((p.n + tm - 1) / tm);
-        return fixed + (tiles + cus - 1) / cus * per_tile;
-    };
-    using Launch = hipError_t (*)(const BlockParams &, hipStream_t);
-    const std::pair<int64_t, Launch> tiles[] = {
-        {cost(128, 128, 45, 515), launch_tile<128, 128, 32>},
-        {cost(128, 64, 40, 281), launch_tile<128, 64, 32>},
-        {cost(64, 64, 25, 147), launch_tile<64, 64, 64>},
-        {cost(64, 32, 33, 77), launch_tile<64, 32, 64>},
-        {cost(32, 32, 10, 44), launch_tile<32, 32, 128>},
-    };
+    auto count = [&](int tm, int tn) { return ((out + tn - 1) / tn) * ((n + tm - 1) / tm); };
     // past 8192 tiles of 128 x 128 (32 rounds) a last round is a few percent,
     // and the grids of smaller tiles could leave the launch limits (65535
     // blocks of rows)
-    const bool many = ((p.out + 127) / 128) * (int64_t)((p.n + 127) / 128) > 8192;
-    const auto least = std::min_element(
-        std::begin(tiles), many ? std::begin(tiles) + 1 : std::end(tiles),
-        [](const auto &a, const auto &b) { return a.first < b.first; });
-    return least->second(p, stream);
+    if (count(128, 128) > 8192)
+        return kTiles[0];
+    auto cost = [&](const Tile &t) {
+        const int64_t rounds = (count(t.m, t.n) + cus - 1) / cus;
+        return (in + t.k - 1) / t.k * (t.fill + rounds * t.round);
+    };
+    return *std::min_element(std::begin(kTiles), std::end(kTiles),
+                             [&](const Tile &a, const Tile &b) { return cost(a) < cost(b); });
 }
 
 // Tokens project_few_kernel takes: from 6 (one wave per row spreads over more
@@ -678,8 +685,16 @@ static hipError_t launch_tiles(const BlockParams &p, hipStream_t stream)
 // 2816 x 4096: 42.7 us against 35.2 us).
 constexpr int kFewFrom = 6, kFewTo = 32;
 
+// Token blocks of a project_few_kernel workgroup.
+static int few_blocks(int64_t n, int64_t out, int64_t cus)
+{
+    const int64_t blocks = (n + 15) / 16;
+    return blocks == 1 || blocks * ((out + 15) / 16) <= cus ? 1 : 2;
+}
+
 hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
 {
+    const int cus = std::max(device_cus(), 1);
     if (p.n < kFewFrom) {
         const dim3 grid((p.out + 3) / 4);
         if (p.n == 1 && p.in % 4 == 0 && p.in <= kLdsRowFloats)
@@ -695,13 +710,13 @@ hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
         else
             project_rows_kernel<5><<<grid, 256, 0, stream>>>(p);
     } else if (p.n <= kFewTo) {
-        const int rows = (p.out + 15) / 16, blocks = (p.n + 15) / 16;
-        if (blocks == 1 || blocks * rows <= device_cus())
-            project_few_kernel<1><<<dim3(rows, blocks), 64 * kFewWaves, 0, stream>>>(p);
+        const int rows = (p.out + 15) / 16;
+        if (few_blocks(p.n, p.out, cus) == 1)
+            project_few_kernel<1><<<dim3(rows, (p.n + 15) / 16), 64 * kFewWaves, 0, stream>>>(p);
         else
             project_few_kernel<2><<<rows, 64 * kFewWaves, 0, stream>>>(p);
     } else {
-        const hipError_t e = launch_tiles(p, stream);
+        const hipError_t e = choose_tile(p.n, p.in, p.out, cus).launch(p, stream);
         if (e != hipSuccess)
             return e;
     }
@@ -742,4 +757,14 @@ extern "C" int pcl_attention_output(pcl_context *ctx, const float *attended, int
         return PCL_NON_FINITE_VALUE;
     }
     return PCL_OK;
+}
+
+extern "C" int pcl_debug_projection_form(int64_t n, int64_t in, int64_t out, int cus)
+{
+    if (n < pcl::kFewFrom)
+        return 1;
+    if (n <= pcl::kFewTo)
+        return 16 * pcl::few_blocks(n, out, cus);
+    const pcl::Tile &t = pcl::choose_tile(n, in, out, std::max(cus, 1));
+    return 1000 * t.m + t.n;
 }

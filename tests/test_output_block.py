@@ -4,8 +4,8 @@ and residual, src/engine/attention.rs:866-884.
 CPU tests pin the oracle's p9_ref_matvec and p9_ref_add restatements with the
 reference's known answers (src/kernels/reference/tests.rs:14-19, 67-73) and
 with the f64-accumulation property the reference tests for its projections
-(tests.rs:21-47: 2^24 + 1 - 2^24 keeps the 1). GPU tests compare both
-projection kernels (few tokens: row streaming; many tokens: f64 MFMA tiles)
+(tests.rs:21-47: 2^24 + 1 - 2^24 keeps the 1). GPU tests compare the
+projection kernels (a wave per row; f64 MFMAs for few tokens; f64 MFMA tiles)
 and the fused post-norm with the oracle.
 """
 import numpy as np
@@ -78,7 +78,8 @@ def run_block(torch, ctx, x, w, scale, res, eps=1e-6, in_place=False):
     return proj.cpu().numpy(), out.cpu().numpy(), err
 
 
-# n = 1, 5, 7, 16, 17, 32, 33: few tokens; 200, 300: f64 MFMA tiles. One token
+# n = 1 and 5: a wave per output row; 7, 16, 17, 32: the few-token kernel; 33,
+# 200, 300: f64 MFMA tiles. One token
 # with input rows of at most 16384 columns (a multiple of 4) is projected
 # with the input row staged in LDS: rows of 1000 (fewer than 4096 columns),
 # 5000 (4096 and a partial step), 4000 (one 4096-column step taken by some
@@ -112,21 +113,46 @@ def test_output_block_matches_the_oracle(torch, ctx, oracle, case):
     assert same >= 0.999 * n * rows
 
 
-# Tiles: 17-40 tokens of 127 or 130 columns take 32 x 32 ones, with
-# remainders of rows and tokens; 520 x 2816: 64 x 32 or 64 x 64; 530 tokens
-# over 4220 rows: 128 x 64; 1400 over 2816: 128 x 128 (the choice follows the
-# device's CU count). Columns below, at and past each K step. The few-token
-# kernel (columns a multiple of 4): 16, 32 and 64 tokens a group and one past
-# each, both ends of its range, output rows of 16 and one past, columns
-# within one wave's 32, one past a 256-column step and past two.
+# (tokens, columns, output rows) and the form they take on 256 CUs: a wave per
+# output row (1), the few-token kernel with 16 or 32 tokens a workgroup, or
+# output tiles of tokens x rows (tokens * 1000 + rows). Per tile shape: a
+# remainder of tokens and rows, columns below one K step, and more than two K
+# steps with a remainder. The few-token kernel: one to 32 tokens around its
+# blocks of 16, output rows of 16 and one past, columns within one wave's 16,
+# at and past 256-column steps, and remainders of a quad; enough rows for
+# two blocks a workgroup.
+FORMS = {
+    (3, 4, 1): 1, (4, 28, 16): 1, (5, 4096, 2816): 1, (3, 1001, 77): 1, (5, 1003, 33): 1,
+    (6, 4, 1): 16, (13, 1001, 77): 16, (16, 260, 17): 16, (17, 256, 33): 16, (31, 126, 32): 16,
+    (17, 127, 33): 16, (32, 516, 16): 16, (31, 770, 4100): 32, (32, 1024, 2816): 32,
+    (33, 512, 40): 32032, (40, 130, 65): 32032, (64, 1028, 31): 32032, (65, 772, 33): 32032,
+    (128, 96, 18): 32032, (129, 68, 2816): 32032, (200, 381, 2816): 32032,
+    (530, 34, 4220): 64032, (480, 200, 2816): 64032, (497, 261, 2801): 64032,
+    (65, 96, 4220): 32032,
+    (700, 63, 2816): 64064, (700, 330, 2816): 64064, (300, 199, 2803): 64064,
+    (520, 65, 2816): 128064, (2100, 101, 2816): 128064,
+    (1400, 31, 2816): 128128, (1400, 133, 2816): 128128, (1301, 98, 2790): 128128,
+}
+
+
+def test_projection_forms(pcl):
+    form = pcl.load().pcl_debug_projection_form
+    for case, want in FORMS.items():
+        assert form(*case, 256) == want, case
+    # the column count decides between shapes: whole K steps of 32 for narrow
+    # rows (2000 x 96: 39 us in 128 x 64, 49 us in 64 x 32), less padding of
+    # tokens for wide ones
+    assert form(2000, 96, 2816, 256) == 128064 and form(2000, 4096, 2816, 256) == 64032
+    assert form(520, 64, 2816, 256) in (64064, 64032, 128064)
+    assert form(1, 4096, 2816, 256) == 1 and form(33, 4096, 2816, 0) // 1000 >= 32
+    # sizes at the entry's limits stay within a grid's 65535 blocks of rows
+    assert form(1 << 22, 1 << 20, 1 << 20, 256) == 128128
+    for n, out in ((1 << 22, 16), (1 << 22, 1 << 20), (1 << 20, 128)):
+        assert n / (form(n, 64, out, 256) // 1000) <= 65535
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", [(17, 127, 33), (31, 126, 32), (40, 130, 65), (129, 68, 2816),
-                                  (520, 65, 2816), (700, 63, 2816), (530, 34, 4220),
-                                  (1400, 31, 2816),
-                                  (3, 4, 1), (4, 28, 16), (16, 260, 17), (17, 256, 33),
-                                  (32, 516, 16), (33, 512, 40), (64, 1028, 31), (65, 772, 33),
-                                  (128, 96, 18), (65, 96, 4220), (5, 4096, 2816)],
-                         ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("case", FORMS, ids=lambda c: "x".join(map(str, c)))
 def test_projection_matches_f64_sums(torch, ctx, case):
     n, cols, rows = case
     g = np.random.default_rng(sum(case))
@@ -177,7 +203,8 @@ def test_one_token_projection_equals_the_multi_token_one_bitwise(torch, ctx, col
                                   (6, 1028, 33), (8, 4098, 17), (16, 260, 64), (16, 1, 1), (17, 4096, 130),
                                   (31, 1003, 48), (32, 512, 4200), (17, 259, 2816), (32, 3, 4200),
                                   (34, 4097, 33), (64, 1028, 300), (128, 196, 65),
-                                  (200, 1000, 2816), (520, 515, 2816), (700, 261, 2816),
+                                  (200, 1000, 2816), (480, 200, 2816), (520, 515, 2816),
+                                  (700, 261, 2816),
                                   (1400, 133, 2816), (2100, 130, 2816)],
                          ids=lambda c: "x".join(map(str, c)))
 def test_a_tokens_projection_does_not_depend_on_the_token_count(torch, ctx, case):
