@@ -233,6 +233,12 @@ int pcl_context_sync(pcl_context *ctx, int *device_error);
 /* Kernel the descriptor resolves to under PCL_KERNEL_AUTO. */
 int pcl_attention_resolve_kernel(const pcl_attention_desc *desc);
 
+/* For tests: the (query, head) rows of one KV head that a workgroup of the
+ * tiled kernels owns when pcl_attention_launch runs this descriptor on a
+ * device of `cus` compute units; 0 when it takes another kernel, -1 when it
+ * is rejected. */
+int pcl_debug_tiled_rows(const pcl_attention_desc *desc, int cus);
+
 /* Bound of the spread decode's waits for the scores of the other
  * workgroups of a key chunk, in polls of a few hundred cycles each; 0
  * restores the default (65536, some tens of milliseconds). A wave whose wait

@@ -59,6 +59,7 @@ EXPORTS = (
     "pcl_context_reserve",
     "pcl_context_sync",
     "pcl_attention_resolve_kernel",
+    "pcl_debug_tiled_rows",
     "pcl_context_set_wait_limit",
     "pcl_debug_set_epoch_counter",
     "pcl_context_set_timing",
@@ -179,6 +180,8 @@ def load():
     lib.pcl_context_sync.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
     lib.pcl_attention_resolve_kernel.restype = ctypes.c_int
     lib.pcl_attention_resolve_kernel.argtypes = [ctypes.POINTER(PclDesc)]
+    lib.pcl_debug_tiled_rows.restype = ctypes.c_int
+    lib.pcl_debug_tiled_rows.argtypes = [ctypes.POINTER(PclDesc), ctypes.c_int]
     lib.pcl_context_set_wait_limit.restype = ctypes.c_int
     lib.pcl_context_set_wait_limit.argtypes = [vp, ctypes.c_int]
     lib.pcl_context_set_timing.restype = ctypes.c_int

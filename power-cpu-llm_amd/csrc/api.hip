@@ -21,6 +21,7 @@ hipError_t launch_spread_kv(const Params &p, hipStream_t stream);
 int tiled_rows(int dk);
 int spread_slices(int dk);
 int device_cus();
+int tiled_block_rows(const Params &p, int64_t cus);
 // published score words (64-bit) of one spread item: 16 key blocks x 4 x 64
 // lanes
 constexpr size_t kSpreadWordsPerItem = 2 * kTilesPerChunk * 4 * 64;
@@ -873,6 +874,21 @@ int pcl_attention_resolve_kernel(const pcl_attention_desc *desc)
                   &plan) != PCL_OK)
         return -1;
     return plan.kernel;
+}
+
+int pcl_debug_tiled_rows(const pcl_attention_desc *desc, int cus)
+{
+    if (!desc || desc->kvheads <= 0)
+        return -1;
+    const int64_t group = desc->qheads / desc->kvheads;
+    Plan plan;
+    if (make_plan(*desc, desc->kh_first * group, desc->kh_end * group, desc->kh_first * group,
+                  &plan) != PCL_OK)
+        return -1;
+    if (plan.empty || (plan.kernel != PCL_KERNEL_TILED && plan.kernel != PCL_KERNEL_TILED_SPLIT))
+        return 0;
+    return plan.kernel == PCL_KERNEL_TILED ? pcl::tiled_block_rows(plan.p, std::max(cus, 1))
+                                           : pcl::tiled_rows(plan.p.dk);
 }
 
 } // extern "C"

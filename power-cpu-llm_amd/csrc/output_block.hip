@@ -659,7 +659,7 @@ constexpr Tile kTiles[] = {
 // 60 us, 256 tokens 581 -> 139 us, 1000 tokens 589 -> 421 us, 2000 tokens 1076
 // -> 783 us, 4096 tokens 1.62 -> 1.49 ms (0.81 of the fp64 MFMA peak); 2000
 // tokens of 96 columns 44 -> 38 us (49 us by a rule without the column count).
-const Tile &choose_tile(int64_t n, int64_t in, int64_t out, int64_t cus)
+static const Tile &choose_tile(int64_t n, int64_t in, int64_t out, int64_t cus)
 {
     auto count = [&](int tm, int tn) { return ((out + tn - 1) / tn) * ((n + tm - 1) / tm); };
     // past 8192 tiles of 128 x 128 (32 rounds) a last round is a few percent,

@@ -577,35 +577,86 @@ static int64_t block_tiles(const Params &p, int64_t fa, int64_t rows)
     return std::max<int64_t>((k_hi + kTile - 1) / kTile - k_lo / kTile, 0);
 }
 
-// Tiles of the CU with the most, over row blocks of `rows` dealt last block
-// first: at least the mean, and at least k + 1 of the k * cus + 1 longest
-// blocks (which the dealing comes close to).
-int64_t span_tiles(const Params &p, int64_t rows, int64_t cus)
+// Key tiles of the i-th of the row blocks of `rows` rows as they are dealt:
+// the last block of every KV head first.
+static int64_t dealt_tiles(const Params &p, int64_t rows, int64_t i)
+{
+    const int64_t qb = (p.nrows + rows - 1) / rows - 1 - i / p.nkv;
+    return qb < 0 ? 0 : block_tiles(p, qb * rows, rows);
+}
+
+// Hundredths of a tile that a CU works on average, blocks costing `extra` more
+// for their start and end.
+static int64_t mean_tiles(const Params &p, int64_t rows, int64_t cus, int64_t extra)
 {
     const int64_t nqb = (p.nrows + rows - 1) / rows;
-    int64_t total = 0, span = 0;
+    int64_t sum = 0;
     for (int64_t qb = 0; qb < nqb; ++qb)
-        total += block_tiles(p, qb * rows, rows) * p.nkv;
-    for (int64_t k = 0; k * cus < nqb * p.nkv; ++k)
-        span = std::max(span, (k + 1) * block_tiles(p, (nqb - 1 - k * cus / p.nkv) * rows, rows));
-    return std::max(span, (total + cus - 1) / cus);
+        sum += 100 * block_tiles(p, qb * rows, rows) + extra;
+    return sum * p.nkv / cus;
+}
+
+// Hundredths of a tile until the last CU ends, one block at a time on each:
+// the longest block, or the mean, or a block of a later round behind the
+// shortest of each round before it. `last`: percent of a tile's time that the
+// last block's tiles take.
+int64_t span_tiles(const Params &p, int64_t rows, int64_t cus, int64_t extra, int64_t last)
+{
+    const int64_t blocks = (p.nrows + rows - 1) / rows * p.nkv;
+    int64_t span = std::max(last * dealt_tiles(p, rows, 0), 100 * dealt_tiles(p, rows, p.nkv));
+    int64_t before = 0;
+    for (int64_t i = cus; i < blocks; i += cus) {
+        before += 100 * dealt_tiles(p, rows, i - 1) + extra;
+        span = std::max(span, before + 100 * dealt_tiles(p, rows, i));
+    }
+    return std::max(span + extra, mean_tiles(p, rows, cus, extra));
 }
 
 // Whether 64-row blocks (four waves, one per SIMD) end sooner than 128-row
 // ones. A CU runs a 64-row tile in 0.68 of a 128-row one's time (one wave
-// hides less of its own latency), and several rounds of unequal blocks end
-// up to 15 % past their mean: 0.78 of the tiles must be less. Where one round
-// holds every block the longest decides, and half of it is always less. At
-// head dim 64 two such blocks share a CU, so the mean counts half.
-// Measured, causal prompts of 16 query and 8 KV heads of 256 dims, 128 rows
-// against 64: 1024 tokens 308 -> 209 us, 2048 611 -> 445 us, 2560 765 -> 749
-// us, 1024 over 5000 keys 1491 -> 989 us; 3001 tokens 896 against 1011 us and
-// 4096 1308 against 1686 us keep 128 rows.
-template <int DK> static bool half_blocks(const Params &p)
+// hides less of its own latency), a block's start and end cost about two
+// tiles, and rounds of unequal blocks end past their mean: 0.78 of the span
+// must be less (0.80 at head dim 128 in several rounds). A 128-row block whose
+// last 64 rows are absent takes 0.55 of a whole one's time (one wave a SIMD
+// works), so short prompts of one query head per KV head keep it. Measured,
+// causal prompts of 16 query and 8 KV heads of 256 dims, 128 rows against 64:
+// 1024 tokens 308 -> 209 us, 2048 611 -> 450 us, 1024 over 5000 keys 1491 ->
+// 989 us; 3001 tokens 896 against 1011 us and 4096 1308 against 1686 us keep
+// 128 rows. 8 query and 8 KV heads, 181 tokens: 42.4 against 46.7 us, kept.
+//
+// At head dim 64 two blocks of either size share a CU. One round of 64-row
+// blocks is as above; where they take two and 128-row ones one, 0.58 of the
+// span must be less; where 128-row blocks take two rounds (both resident), the
+// first CU's blocks in turn stand for the span, 0.55 of it; and past that the
+// 64-row blocks only add starts and ends (8192 tokens, window 1024, 16 heads:
+// 362 against 431 us). 4 KV heads of 4 query heads: 1024 tokens 96 -> 70 us,
+// 2500 247 -> 198 us, 3600 398 -> 351 us; window 1024 at 3600 tokens keeps 128
+// rows (178 against 184 us), and so do 4096 tokens, 7 % to the worse: a bound
+// that takes them takes others that are up to 13 % slower. Of 551 sizes at
+// head dim 64 three are slower than in 128 rows, by up to 4 %; of 833 at 128
+// and 256 none.
+static bool half_blocks(const Params &p, int64_t cus)
 {
-    constexpr int kPercent = DK == 64 ? 55 : 78;
-    const int64_t cus = std::max(device_cus(), 1);
-    return kPercent * span_tiles(p, kTiledRows / 2, cus) < 100 * span_tiles(p, kTiledRows, cus);
+    constexpr int64_t kWhole = kTiledRows, kHalf = kTiledRows / 2;
+    const int64_t nqb = (p.nrows + kWhole - 1) / kWhole;
+    const int64_t wholes = nqb * p.nkv, halves = (p.nrows + kHalf - 1) / kHalf * p.nkv;
+    const int64_t last = p.nrows - (nqb - 1) * kWhole <= kHalf ? 55 : 100;
+    if (p.dk == 64 && wholes > 2 * cus)
+        return false;
+    if (p.dk == 64 && wholes > cus) {
+        int64_t half = 0;
+        for (int64_t i = 0; i < halves; i += cus)
+            half += 100 * dealt_tiles(p, kHalf, i) + 100;
+        const int64_t whole =
+            100 * dealt_tiles(p, kWhole, 0) + 70 * dealt_tiles(p, kWhole, cus);
+        return 55 * std::max(half, mean_tiles(p, kHalf, cus, 100)) <
+               100 * std::max(whole, mean_tiles(p, kWhole, cus, 0));
+    }
+    const int64_t extra = p.dk == 64 ? 300 : 200;
+    const int64_t percent = p.dk == 64 ? (halves <= cus ? 82 : 58)
+                                     : p.dk == 128 && wholes > cus ? 80 : 78;
+    return percent * span_tiles(p, kHalf, cus, extra, 100) <
+           100 * span_tiles(p, kWhole, cus, extra, last);
 }
 
 template <int DK>
@@ -613,7 +664,7 @@ static hipError_t launch_tiled_dk(const Params &p, int split, hipStream_t stream
 {
     const int nqb = (p.nrows + kTiledRows - 1) / kTiledRows;
     const int tail = split ? tiled_tail_chunks(p, nqb, device_cus()) : 0;
-    if (!split && half_blocks<DK>(p)) {
+    if (!split && half_blocks(p, std::max(device_cus(), 1))) {
         constexpr int W = kTiledWaves / 2;
         const dim3 half((p.nrows + W * kRows - 1) / (W * kRows) * p.nkv);
         return p.softcap > 0.0f ? launch_tiled_grid<DK, W, true>(p, 0, half, stream)
@@ -642,6 +693,15 @@ int tiled_wide_rows();
 int tiled_rows(int dk)
 {
     return dk > 256 ? tiled_wide_rows() : kTiledRows;
+}
+
+bool wide_half_blocks(const Params &p, int64_t cus);
+
+// Rows of one workgroup of an unsplit launch on `cus` compute units.
+int tiled_block_rows(const Params &p, int64_t cus)
+{
+    const bool half = p.dk > 256 ? wide_half_blocks(p, cus) : half_blocks(p, cus);
+    return tiled_rows(p.dk) / (half ? 2 : 1);
 }
 
 // *merged: set when the launch itself wrote the merged output of a split

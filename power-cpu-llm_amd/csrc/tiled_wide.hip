@@ -534,20 +534,21 @@ static hipError_t launch_wide(const Params &p, int split, dim3 grid, hipStream_t
 
 int device_cus();
 int tiled_tail_chunks(const Params &p, int nqb, int cus);
-int64_t span_tiles(const Params &p, int64_t rows, int64_t cus);
+int64_t span_tiles(const Params &p, int64_t rows, int64_t cus, int64_t extra, int64_t last);
 hipError_t launch_fan_chunk(const Params &p, int ci, bool merge_out, hipStream_t stream);
 
 // Whether 32-row blocks (two units, one wave per SIMD) end sooner than
 // 64-row ones: with fewer tiles on the busiest CU, or one round of blocks
 // either way. A SIMD's two waves take turns on the score chains, so half the
 // rows save less here than at head dim 256: a 32-row tile takes 0.9 of a
-// 64-row one's time. Causal prompts of 16 query and 2 KV heads, 64 rows
+// 64-row one's time, and a bound of 0.95 told the two apart without a miss at
+// 360 sizes (0.9 missed three by up to 7 %). Causal prompts of 16 query and 2 KV heads, 64 rows
 // against 32: 128 tokens 53.7 -> 48.2 us, 512 tokens 181 -> 163 us, 768 tokens
 // 266 -> 241 us, 1024 tokens 352 -> 349 us.
-static bool wide_half_blocks(const Params &p)
+bool wide_half_blocks(const Params &p, int64_t cus)
 {
-    const int64_t cus = std::max(device_cus(), 1);
-    return 95 * span_tiles(p, kWideRows / 2, cus) < 100 * span_tiles(p, kWideRows, cus);
+    return 95 * span_tiles(p, kWideRows / 2, cus, 0, 100) <
+           100 * span_tiles(p, kWideRows, cus, 0, 100);
 }
 
 // A split launch whose chunk items leave a small last round runs that
@@ -558,7 +559,7 @@ hipError_t launch_tiled_wide(const Params &p, int split, hipStream_t stream, boo
 {
     const int nqb = (p.nrows + kWideRows - 1) / kWideRows;
     const int tail = split ? tiled_tail_chunks(p, nqb, device_cus()) : 0;
-    if (!split && wide_half_blocks(p)) {
+    if (!split && wide_half_blocks(p, std::max(device_cus(), 1))) {
         constexpr int U = kWideUnits / 2;
         const dim3 half((p.nrows + U * kRows - 1) / (U * kRows) * p.nkv);
         return p.softcap > 0.0f ? launch_wide<U, true>(p, 0, half, stream)

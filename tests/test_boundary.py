@@ -79,6 +79,42 @@ def test_raw_entries_reject_geometry_before_device_work(pcl):
     assert not pcl.raw_multi_kv(one, 1, 16, one, one, 2, 1, 16, 1, None, 1, 32, 0, 1)[0]
 
 
+def tiled_rows(pcl, qheads, kvheads, dim, nq, nkeys, window=0, causal=1, cus=256):
+    d = pcl.Context.desc(q=16, q_stride=qheads * dim, nq=nq, k0=16, v0=16, n0=nkeys,
+                         qheads=qheads, kvheads=kvheads, dim=dim, kh_first=0, kh_end=kvheads,
+                         causal=causal, window=window, first_query=nkeys - nq, out=16,
+                         o_stride=qheads * dim)
+    return pcl.load().pcl_debug_tiled_rows(ctypes.byref(d), cus)
+
+
+def test_row_blocks_follow_the_measured_times(pcl):
+    # 64-row blocks where they end sooner on 256 CUs, 128-row ones where not
+    for case in [(16, 8, 256, 1024, 1024), (16, 8, 256, 2048, 2048), (16, 8, 256, 1024, 5000),
+                 (32, 8, 128, 512, 512), (32, 32, 128, 100, 100), (16, 4, 64, 1024, 1024),
+                 (16, 4, 64, 2500, 2500), (16, 4, 64, 3600, 3600), (16, 8, 256, 65, 65)]:
+        assert tiled_rows(pcl, *case) == 64, case
+    for case in [(16, 8, 256, 4096, 4096), (16, 8, 256, 3001, 3001),
+                 (16, 8, 256, 3001, 3001, 1024),
+                 # the last block holds at most 64 rows: one query head per KV head
+                 (32, 32, 128, 64, 64), (32, 32, 128, 181, 181), (16, 16, 64, 64, 64),
+                 (16, 16, 64, 181, 181), (8, 8, 256, 64, 64), (8, 8, 256, 181, 181),
+                 # short blocks of a window in several rounds
+                 (16, 8, 256, 1200, 1200, 256), (16, 16, 128, 1200, 1200, 256),
+                 (16, 4, 64, 3600, 3600, 1024), (16, 4, 64, 2500, 2500, 512),
+                 (16, 16, 64, 8192, 8192, 1024), (16, 16, 64, 4096, 4096, 512),
+                 (12, 4, 48, 5000, 5000, 256)]:
+        assert tiled_rows(pcl, *case) == 128, case
+    assert tiled_rows(pcl, 16, 2, 512, 512, 512) == 32
+    assert tiled_rows(pcl, 16, 2, 512, 4096, 4096) == 64
+    # a canvas of few blocks splits over chunks in whole blocks; a decode does
+    # not take the tiled kernels; fewer CUs make more rounds
+    assert tiled_rows(pcl, 16, 8, 256, 256, 2304, 0, 0) == 128
+    assert tiled_rows(pcl, 16, 8, 256, 1, 1024) == 0
+    assert tiled_rows(pcl, 16, 8, 256, 1024, 1024, cus=64) == 128
+    assert tiled_rows(pcl, 16, 8, 256, 1024, 1024, cus=0) in (64, 128)
+    assert tiled_rows(pcl, 16, 0, 256, 1024, 1024) == -1
+
+
 def test_descriptor_validation_on_the_host(pcl):
     # workspace sizing and kernel choice run on the host only
     d = pcl.Context.desc(q=16, q_stride=16 * 256, nq=1, k0=16, v0=16, n0=32768, qheads=16,
