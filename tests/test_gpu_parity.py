@@ -6,6 +6,7 @@ max-abs with the same argmax per (query, head) row, and checks the
 size-independent properties the design promises (every kernel gives the
 same bits; head, query and KV-head ranges do not change results).
 """
+import ctypes
 import math
 import os
 
@@ -771,21 +772,27 @@ def test_explicit_masks_segments_scale_and_kv_ranges_keep_bits(torch, ctx):
                                                                 6 * group * dim]))
 
 
-# (qheads, kvheads, dim, queries, keys, causal, window): rows one below, at and
-# past 64- and 128-row blocks; one round of blocks (64 rows each), many equal
-# blocks (128 rows each), windows inside key chunks, a padded head dim.
-ROW_BLOCK_CASES = [(2, 1, 256, 31, 300, 1, 0), (2, 1, 256, 32, 300, 1, 0),
-                   (16, 8, 256, 65, 65, 1, 0), (16, 8, 256, 1087, 1087, 1, 500),
-                   (32, 8, 128, 33, 700, 1, 0), (16, 4, 64, 400, 900, 1, 0),
-                   (16, 4, 64, 517, 517, 1, 100), (4, 2, 208, 49, 333, 1, 0),
-                   (16, 8, 256, 2048, 288, 0, 0), (16, 2, 512, 40, 600, 1, 0),
-                   (16, 2, 512, 517, 517, 1, 100), (8, 1, 400, 21, 290, 1, 0)]
+# (qheads, kvheads, dim, queries, keys, causal, window) and the rows of a
+# workgroup on 256 CUs: rows one below, at and past 64- and 128-row blocks, one
+# round of blocks, windows inside key chunks, padded head dims; the whole
+# blocks' own cases are below.
+ROW_BLOCK_CASES = {(2, 1, 256, 31, 300, 1, 0): 128, (2, 1, 256, 32, 300, 1, 0): 128,
+                   (16, 8, 256, 65, 65, 1, 0): 64, (16, 8, 256, 1087, 1087, 1, 500): 64,
+                   (32, 8, 128, 33, 700, 1, 0): 64, (16, 4, 64, 400, 900, 1, 0): 64,
+                   (16, 4, 64, 517, 517, 1, 100): 64, (4, 2, 208, 49, 333, 1, 0): 64,
+                   (16, 8, 256, 2048, 288, 0, 0): 128, (16, 2, 512, 40, 600, 1, 0): 32,
+                   (16, 2, 512, 517, 517, 1, 100): 32, (8, 1, 400, 21, 290, 1, 0): 32}
+
+
+def block_rows(torch, pcl, desc):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return pcl.load().pcl_debug_tiled_rows(ctypes.byref(desc), cus)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("softcap", [0.0, 3.0])
 @pytest.mark.parametrize("case", ROW_BLOCK_CASES, ids=lambda c: "x".join(map(str, c)))
-def test_row_blocks_keep_the_split_kernels_bits(torch, ctx, case, softcap):
+def test_row_blocks_keep_the_split_kernels_bits(torch, pcl, ctx, case, softcap):
     qheads, kvh, dim, nq, nkeys, causal, window = case
     q = gpu_normals(torch, 0x5EED0811, (nq, qheads, dim)) * (1.0 / 16.0)
     k = gpu_normals(torch, 0x5EED0812, (nkeys, kvh, dim))
@@ -802,6 +809,65 @@ def test_row_blocks_keep_the_split_kernels_bits(torch, ctx, case, softcap):
         ctx.launch(d)
         assert ctx.sync() == 0
         outs.append(out.cpu().numpy())
+    assert block_rows(torch, pcl, d) == ROW_BLOCK_CASES[case]
+    assert np.array_equal(bits(outs[0]), bits(outs[1]))
+
+
+# Launches of whole blocks (128 rows, 64 at head dim 512): equal blocks of
+# about one round of 256 CUs, windowed and ragged prompts of several rounds,
+# a half-empty last block; padded head dims, more than one span of 4096 keys,
+# two key segments, a KV-head sub-range and explicit masks. (qheads, kvheads,
+# dim, queries, keys of the first segment, of the second, causal, window, KV
+# heads, masked)
+FULL_BLOCK_CASES = [
+    (16, 8, 256, 2048, 288, 0, 0, 0, None, False), (16, 8, 208, 2041, 300, 33, 0, 0, None, False),
+    (16, 8, 256, 2048, 4200, 100, 0, 0, None, False),
+    (12, 6, 256, 3501, 250, 70, 0, 0, (1, 6), False),
+    (16, 8, 256, 2048, 400, 40, 0, 0, None, True),
+    (16, 8, 256, 3001, 3001, 0, 1, 300, None, False), (8, 8, 256, 53, 53, 0, 1, 0, None, False),
+    (8, 8, 144, 181, 181, 0, 1, 0, None, False), (16, 8, 128, 2048, 288, 0, 0, 0, None, False),
+    (16, 8, 112, 2045, 500, 19, 0, 0, (2, 8), False),
+    (16, 8, 128, 2048, 4200, 0, 0, 0, None, False),
+    (32, 8, 128, 1100, 1100, 0, 1, 300, None, False), (16, 8, 80, 2048, 320, 0, 0, 0, None, True),
+    (16, 4, 64, 2048, 700, 61, 0, 0, None, False), (12, 4, 48, 3600, 3600, 0, 1, 256, None, False),
+    (16, 4, 64, 2048, 4500, 0, 0, 0, None, True), (16, 16, 64, 181, 181, 0, 1, 0, None, False),
+    (16, 2, 512, 1024, 288, 0, 0, 0, None, False), (16, 2, 400, 1021, 300, 41, 0, 0, None, False),
+    (16, 2, 512, 1024, 4200, 64, 0, 0, None, False), (16, 2, 512, 1024, 500, 0, 0, 0, None, True),
+    (24, 3, 512, 1100, 333, 0, 0, 0, (1, 3), False),
+    (16, 2, 512, 2100, 2100, 0, 1, 300, None, False),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("softcap", [0.0, 3.0])
+@pytest.mark.parametrize("case", FULL_BLOCK_CASES, ids=lambda c: "-".join(map(str, c)))
+def test_whole_row_blocks_keep_the_split_kernels_bits(torch, pcl, ctx, case, softcap):
+    qheads, kvh, dim, nq, n0, n1, causal, window, kv, masked = case
+    kv = kv or (0, kvh)
+    group = qheads // kvh
+    q = gpu_normals(torch, 0x5EED0821, (nq, qheads, dim)) * (1.0 / 16.0)
+    k = gpu_normals(torch, 0x5EED0822, (n0 + n1, kvh, dim))
+    v = gpu_normals(torch, 0x5EED0823, (n0 + n1, kvh, dim))
+    k1, v1 = k[n0:].clone(), v[n0:].clone()
+    kw = {}
+    if masked:
+        mask = (gpu_normals(torch, 0x5EED0824, (nq, n0 + n1)) < 0.5).to(torch.uint8)
+        mask[:, -1] = 1
+        kw = dict(mask=mask.data_ptr(), mask_stride=n0 + n1)
+    outs = []
+    for kernel in (1, 2):
+        out = torch.full((nq, (kv[1] - kv[0]) * group, dim), float("nan"), device="cuda:0")
+        d = ctx.desc(q=q.data_ptr(), q_stride=qheads * dim, nq=nq, k0=k.data_ptr(),
+                     v0=v.data_ptr(), n0=n0, k1=k1.data_ptr() or None, v1=v1.data_ptr() or None,
+                     n1=n1, qheads=qheads, kvheads=kvh, dim=dim, kh_first=kv[0], kh_end=kv[1],
+                     causal=causal, window=window, first_key=0, first_query=max(n0 + n1 - nq, 0),
+                     softcap=softcap, out=out.data_ptr(), o_stride=out.shape[1] * dim,
+                     kernel=kernel, **kw)
+        ctx.reserve(ctx.workspace_bytes(d))
+        ctx.launch(d)
+        assert ctx.sync() == 0
+        outs.append(out.cpu().numpy())
+    assert block_rows(torch, pcl, d) == (64 if dim > 256 else 128)
     assert np.array_equal(bits(outs[0]), bits(outs[1]))
 
 
