@@ -439,7 +439,8 @@ def time_output_workload(torch, pcl, ctx, name, steps, warmup, seed):
     if nq == 1 and width % 4 == 0 and width <= 16384:
         kernel = "project_row_lds"
     else:
-        kernel = "project_rows" if nq <= 32 else "project_tiles"
+        kernel = ("project_rows" if nq <= 5 else "project_few" if nq <= 32 else
+                  "project_tiles")
     return ev, wall, kernel, None, {"stream_ms": ev, "combine_ms": 0.0}, nsets
 
 

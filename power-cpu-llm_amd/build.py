@@ -16,7 +16,8 @@ SOURCES = ["csrc/split_kv.hip", "csrc/pipe_kv.hip", "csrc/spread_kv.hip",
            "csrc/tiled.hip", "csrc/tiled_wide.hip", "csrc/fan_kv.hip",
            "csrc/api.hip", "csrc/kv_cache.hip", "csrc/head_transform.hip",
            "csrc/output_block.hip"]
-HEADERS = ["csrc/attention_device.hpp", "csrc/context.hpp", os.path.join(ROOT, "include", "pcl_attention.h")]
+HEADERS = ["csrc/attention_device.hpp", "csrc/context.hpp", "csrc/launch.hpp",
+           os.path.join(ROOT, "include", "pcl_attention.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -1,6 +1,7 @@
 // Host side of the attention backend: contexts, descriptor validation,
 // kernel choice and the C ABI of include/pcl_attention.h.
 #include "attention_device.hpp"
+#include "launch.hpp"
 #include "pcl_attention.h"
 
 #include <algorithm>
@@ -12,16 +13,6 @@
 #include <vector>
 
 namespace pcl {
-hipError_t launch_split_kv(const Params &p, hipStream_t stream);
-hipError_t launch_combine(const Params &p, hipStream_t stream);
-hipError_t launch_pipe_kv(const Params &p, hipStream_t stream);
-hipError_t launch_tiled(const Params &p, int split, hipStream_t stream, bool *merged);
-hipError_t launch_fan_kv(const Params &p, hipStream_t stream);
-hipError_t launch_spread_kv(const Params &p, hipStream_t stream);
-int tiled_rows(int dk);
-int spread_slices(int dk);
-int device_cus();
-int tiled_block_rows(const Params &p, int64_t cus);
 // published score words (64-bit) of one spread item: 16 key blocks x 4 x 64
 // lanes
 constexpr size_t kSpreadWordsPerItem = 2 * kTilesPerChunk * 4 * 64;

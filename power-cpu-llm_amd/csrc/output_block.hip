@@ -33,6 +33,7 @@
 //     result = residual + y (f32).
 #include "attention_device.hpp"
 #include "context.hpp"
+#include "launch.hpp"
 #include "pcl_attention.h"
 
 #include <algorithm>
@@ -42,10 +43,6 @@
 #include <type_traits>
 
 namespace pcl {
-
-constexpr int kMaxDevices = 64;
-
-int device_cus();
 
 constexpr int kErrBlock = 8; // non-finite value in the output block
 

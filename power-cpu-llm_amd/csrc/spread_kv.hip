@@ -53,6 +53,7 @@
 // instead was measured slower: its chain of dependent round trips outlasted
 // the separate combine launch.)
 #include "attention_device.hpp"
+#include "launch.hpp"
 
 namespace pcl {
 
@@ -588,8 +589,6 @@ __global__ __launch_bounds__(64 * WV, 2) void spread_kv_kernel(Params p)
 // chunk partial goes out as device-coherent words to the merge workgroups
 // appended to the grid (one thread per four dims of a row), which may run
 // on any XCD.
-int device_cus();
-
 constexpr int kWideSlices = 16;  // slices per item: one key block each
 constexpr int kWidePieceU = 4;   // score chain steps (32 dims each) per K piece
 constexpr int kWidePieces = 512 / 32 / kWidePieceU;

@@ -2,8 +2,8 @@
 //
 // One workgroup of 8 waves (two per SIMD) owns 128 flat (query, head) rows of
 // one KV head, one 16-row MFMA unit per wave; launches that 64-row blocks
-// balance better over the CUs run 4 waves (half_blocks). Q^T (MFMA B operands) and the
-// chunk state O stay in registers. K and V tiles of 32 keys are copied
+// balance better over the CUs run 4 waves (half_blocks). Q^T (MFMA B
+// operands) and the chunk state O stay in registers. K and V tiles of 32 keys are copied
 // HBM -> LDS by global_load_lds_dwordx4 (no register staging), double
 // buffered. K rows are stored with their 16-byte chunks XOR-swizzled by
 // (key & 7), so the 16 key rows of an MFMA A operand hit distinct banks
@@ -25,23 +25,20 @@
 // eight waves: more, shorter items fill the CUs; the pipelined decode kernel
 // at head dim 64); each row's arithmetic is the same either way.
 #include "attention_device.hpp"
+#include "launch.hpp"
 
 #include <algorithm>
 #include <atomic>
 
 namespace pcl {
 
-hipError_t launch_pipe_kv_chunks(const Params &p, int c0, int n, bool merge_out,
-                                 hipStream_t stream);
-hipError_t launch_fan_chunk(const Params &p, int ci, bool merge_out, hipStream_t stream);
-bool fan_supported(int dk);
-
 constexpr int kTiledWaves = 8;
 constexpr int kTiledRows = kTiledWaves * kRows; // 128
 
 // LDS of one workgroup: two K/V stages, then the leading 64-dim blocks of
 // the span accumulator (as many as the 160 KiB of a CU hold beside the
-// stages: one at head dim 256, all of them at 128 and 64).
+// stages: one at head dim 256, all of them at 128 and 64), sized for 128 rows;
+// four waves use the first half.
 template <int DK> struct TiledLds {
     static constexpr int tileFloats = kTile * DK;
     static constexpr int stage = 2 * tileFloats; // K then V
@@ -78,9 +75,10 @@ __device__ __forceinline__ bool tile_whole(const Params &p, int row_lo, int row_
     return kmax <= qlo && (p.window == 0 || qhi - kmin < p.window);
 }
 
-// One workgroup per CU (its K/V stages fill the LDS), so at most W / 4 waves
-// per SIMD: each wave may hold 256 VGPRs and more, which the operand
-// double-buffering below uses. W waves per workgroup, one 16-row unit each.
+// W waves per workgroup, one 16-row unit each. At head dims 128 and 256 one
+// workgroup per CU (its stages and span blocks fill the LDS), W / 4 waves per
+// SIMD, so each wave may hold 256 VGPRs and more, which the operand
+// double-buffering below uses; at 64 two workgroups share a CU.
 template <int DK, int W, bool CAP>
 __global__ __launch_bounds__(64 * W, W / 4) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
 void tiled_kernel(Params p, int split, int z0)
@@ -496,8 +494,6 @@ void tiled_kernel(Params p, int split, int z0)
     }
 }
 
-constexpr int kMaxDevices = 64;
-
 // Compute units of the current device (cached per device; callers on other
 // threads with their own contexts may race here, so the cache is atomic).
 int device_cus()
@@ -686,16 +682,11 @@ static hipError_t launch_tiled_dk(const Params &p, int split, hipStream_t stream
     return e;
 }
 
-hipError_t launch_tiled_wide(const Params &p, int split, hipStream_t stream, bool *merged);
-int tiled_wide_rows();
-
 // Rows of one workgroup: 128 up to head dim 256; 64 at 512 (tiled_wide.hip).
 int tiled_rows(int dk)
 {
     return dk > 256 ? tiled_wide_rows() : kTiledRows;
 }
-
-bool wide_half_blocks(const Params &p, int64_t cus);
 
 // Rows of one workgroup of an unsplit launch on `cus` compute units.
 int tiled_block_rows(const Params &p, int64_t cus)

@@ -25,6 +25,7 @@
 // The chunk, span and total merges, split launches and masks follow the
 // other tiled kernel (tiled.hip); each wave merges its own dims.
 #include "attention_device.hpp"
+#include "launch.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -506,20 +507,17 @@ void tiled_wide_half_kernel(Params p, int split, int z0)
     tiled_wide<kWideUnits / 2, CAP>(p, split, z0);
 }
 
-constexpr int kWideMaxDevices = 64;
-
-
 template <int U, bool CAP>
 static hipError_t launch_wide(const Params &p, int split, dim3 grid, hipStream_t stream)
 {
     static_assert(U == kWideUnits || U == kWideUnits / 2);
     constexpr auto kernel = U == kWideUnits ? tiled_wide_kernel<CAP> : tiled_wide_half_kernel<CAP>;
-    static std::atomic<bool> configured[kWideMaxDevices];
+    static std::atomic<bool> configured[kMaxDevices];
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess)
         return e;
-    if (dev < 0 || dev >= kWideMaxDevices)
+    if (dev < 0 || dev >= kMaxDevices)
         return hipErrorInvalidDevice;
     if (!configured[dev].load(std::memory_order_acquire)) {
         e = hipFuncSetAttribute((const void *)kernel,
@@ -532,18 +530,13 @@ static hipError_t launch_wide(const Params &p, int split, dim3 grid, hipStream_t
     return hipGetLastError();
 }
 
-int device_cus();
-int tiled_tail_chunks(const Params &p, int nqb, int cus);
-int64_t span_tiles(const Params &p, int64_t rows, int64_t cus, int64_t extra, int64_t last);
-hipError_t launch_fan_chunk(const Params &p, int ci, bool merge_out, hipStream_t stream);
-
 // Whether 32-row blocks (two units, one wave per SIMD) end sooner than
 // 64-row ones: with fewer tiles on the busiest CU, or one round of blocks
 // either way. A SIMD's two waves take turns on the score chains, so half the
 // rows save less here than at head dim 256: a 32-row tile takes 0.9 of a
 // 64-row one's time, and a bound of 0.95 told the two apart without a miss at
-// 360 sizes (0.9 missed three by up to 7 %). Causal prompts of 16 query and 2 KV heads, 64 rows
-// against 32: 128 tokens 53.7 -> 48.2 us, 512 tokens 181 -> 163 us, 768 tokens
+// 360 sizes (0.9 missed three by up to 7 %). Causal prompts of 16 query and 2
+// KV heads, 64 rows against 32: 128 tokens 53.7 -> 48.2 us, 512 tokens 181 -> 163 us, 768 tokens
 // 266 -> 241 us, 1024 tokens 352 -> 349 us.
 bool wide_half_blocks(const Params &p, int64_t cus)
 {

@@ -200,8 +200,8 @@ def test_one_token_projection_equals_the_multi_token_one_bitwise(torch, ctx, col
 # ones, so that f64 sums in another order differ in their f32 bits.
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", [(3, 4096, 300), (2, 1001, 33), (4, 1000, 300), (5, 8193, 16),
-                                  (6, 1028, 33), (8, 4098, 17), (16, 260, 64), (16, 1, 1), (17, 4096, 130),
-                                  (31, 1003, 48), (32, 512, 4200), (17, 259, 2816), (32, 3, 4200),
+                                  (6, 1028, 33), (8, 4098, 17), (16, 260, 64), (16, 1, 1),
+                                  (17, 4096, 130), (31, 1003, 48), (32, 512, 4200), (17, 259, 2816), (32, 3, 4200),
                                   (34, 4097, 33), (64, 1028, 300), (128, 196, 65),
                                   (200, 1000, 2816), (480, 200, 2816), (520, 515, 2816),
                                   (700, 261, 2816),
