@@ -227,24 +227,64 @@ __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
         const int buf = s & 1;
         if (s + 1 < steps)
             load((s + 1) * TK);
+        if constexpr (kI * kJ == 1) {
+            // A single chain of MFMAs: each would wait for its operands'
+            // conversions, and these for the MFMA before it that still reads
+            // their registers. Operands are read 32 and converted 16 columns
+            // ahead into registers of their own (64 tokens of 4096 columns,
+            // 2816 rows: 57.8 -> 52.5 us).
+            const float *ar = sa + (buf * TM + wm + r16) * kRow + 4 * kq;
+            const float *br = sb + (buf * TN + wn + r16) * kRow + 4 * kq;
+            f4 a[2], b[2];
+            double ca[2][4], cb[2][4];
+            auto read = [&](int kc, int set) {
+                a[set] = *(const f4 *)(ar + kc);
+                b[set] = *(const f4 *)(br + kc);
+            };
+            auto convert = [&](int set) {
 #pragma unroll
-        for (int kc = 0; kc < TK; kc += 16) {
-            // MFMA k slot kq of step j holds column kc + 4 kq + j
-            f4 a[kI], b[kJ];
+                for (int j = 0; j < 4; ++j) {
+                    ca[set][j] = (double)a[set][j];
+                    cb[set][j] = (double)b[set][j];
+                }
+            };
+            read(0, 0);
+            read(16, 1);
+            convert(0);
 #pragma unroll
-            for (int i = 0; i < kI; ++i)
-                a[i] = *(const f4 *)(sa + (buf * TM + wm + 16 * i + r16) * kRow + kc + 4 * kq);
+            for (int kc = 0; kc < TK; kc += 16) {
+                const int set = (kc / 16) & 1;
+                if (kc + 32 < TK)
+                    read(kc + 32, set);
+                if (kc + 16 < TK)
+                    convert(set ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < kJ; ++i)
-                b[i] = *(const f4 *)(sb + (buf * TN + wn + 16 * i + r16) * kRow + kc + 4 * kq);
+                for (int j = 0; j < 4; ++j)
+                    acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ca[set][j], cb[set][j],
+                                                                     acc[0][0], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int kc = 0; kc < TK; kc += 16) {
+                // MFMA k slot kq of step j holds column kc + 4 kq + j
+                f4 a[kI], b[kJ];
 #pragma unroll
                 for (int i = 0; i < kI; ++i)
+                    a[i] = *(const f4 *)(sa + (buf * TM + wm + 16 * i + r16) * kRow + kc + 4 * kq);
 #pragma unroll
-                    for (int jj = 0; jj < kJ; ++jj)
-                        acc[i][jj] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                            (double)a[i][j], (double)b[jj][j], acc[i][jj], 0, 0, 0);
+                for (int i = 0; i < kJ; ++i)
+                    b[i] = *(const f4 *)(sb + (buf * TN + wn + 16 * i + r16) * kRow + kc + 4 * kq);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int i = 0; i < kI; ++i)
+#pragma unroll
+                        for (int jj = 0; jj < kJ; ++jj)
+                            acc[i][jj] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                (double)a[i][j], (double)b[jj][j], acc[i][jj], 0, 0, 0);
+            }
         }
         if (s + 1 < steps)
             store(buf ^ 1); // read last in step s - 1, before that step's barrier
@@ -640,11 +680,11 @@ struct Tile {
     hipError_t (*launch)(const BlockParams &, hipStream_t);
 };
 constexpr Tile kTiles[] = {
-    {128, 128, 32, 49, 369, launch_tile<128, 128, 32>},
-    {128, 64, 32, 30, 198, launch_tile<128, 64, 32>},
-    {64, 64, 64, 37, 203, launch_tile<64, 64, 64>},
-    {64, 32, 64, 42, 104, launch_tile<64, 32, 64>},
-    {32, 32, 128, 30, 126, launch_tile<32, 32, 128>},
+    {128, 128, 32, 52, 366, launch_tile<128, 128, 32>},
+    {128, 64, 32, 30, 196, launch_tile<128, 64, 32>},
+    {64, 64, 64, 38, 201, launch_tile<64, 64, 64>},
+    {64, 32, 64, 43, 102, launch_tile<64, 32, 64>},
+    {32, 32, 128, 19, 122, launch_tile<32, 32, 128>},
 };
 
 // The tile with the least time: 352 tiles of 128 x 128 (2000 tokens, 2816
@@ -653,7 +693,7 @@ constexpr Tile kTiles[] = {
 // sizes timed in every shape the choice is 0.6 % from the best on average.
 // Projection of 2816 rows of 4096 columns, 128 x 128 alone (its loads
 // branching over rows and columns) against the chosen tile: 33 tokens 568 ->
-// 60 us, 256 tokens 581 -> 139 us, 1000 tokens 589 -> 421 us, 2000 tokens 1076
+// 53 us, 256 tokens 581 -> 126 us, 1000 tokens 589 -> 421 us, 2000 tokens 1076
 // -> 783 us, 4096 tokens 1.62 -> 1.49 ms (0.81 of the fp64 MFMA peak); 2000
 // tokens of 96 columns 44 -> 38 us (49 us by a rule without the column count).
 static const Tile &choose_tile(int64_t n, int64_t in, int64_t out, int64_t cus)
