@@ -378,12 +378,12 @@ __global__ __launch_bounds__(256) void post_norm_kernel(BlockParams p)
 // The largest input row project_row_lds_kernel stages (64 KiB of LDS).
 constexpr int kLdsRowFloats = 16384;
 
-// One token (p.in % 4 == 0, p.in <= kLdsRowFloats), one wave per output
+// One token, t0 (p.in % 4 == 0, p.in <= kLdsRowFloats), one wave per output
 // row as in project_rows_kernel<1> (the same f64 sums in the same order):
 // the workgroup stages the input row in LDS once, its first 4096 columns
 // requested before the rows' first weights so that the LDS stores wait only
 // for them.
-__global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p)
+__global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p, int t0)
 {
     extern __shared__ f4 xs[];
     const int lane = threadIdx.x & 63;
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p)
     const bool live = r < p.out;
     // a wave past the last row streams row 0 (in bounds; unused)
     const float *wr = p.w + (int64_t)(live ? r : 0) * p.in;
-    const float *xr = p.x;
+    const float *xr = p.x + (int64_t)t0 * p.in;
     f4 wv[16];
     int v = lane;
     if (vecs >= 1024) {
@@ -447,7 +447,7 @@ __global__ __launch_bounds__(256) void project_row_lds_kernel(BlockParams p)
     for (int o = 32; o >= 1; o >>= 1)
         acc += __shfl_xor(acc, o);
     if (lane == 0)
-        stg(p.proj + r, (float)acc);
+        stg(p.proj + (int64_t)t0 * p.out + r, (float)acc);
 }
 
 // The 4 x 4 transpose of four registers over a wave's four 16-lane groups:
@@ -735,7 +735,7 @@ hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
     if (p.n < kFewFrom) {
         const dim3 grid((p.out + 3) / 4);
         if (p.n == 1 && p.in % 4 == 0 && p.in <= kLdsRowFloats)
-            project_row_lds_kernel<<<grid, 256, p.in * 4, stream>>>(p);
+            project_row_lds_kernel<<<grid, 256, p.in * 4, stream>>>(p, 0);
         else if (p.n == 1)
             project_rows_kernel<1><<<grid, 256, 0, stream>>>(p);
         else if (p.n == 2)

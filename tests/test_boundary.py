@@ -274,6 +274,11 @@ def _resource_remarks(source):
     ("fan_kv.hip", "_ZN3pcl13fan_kv_kernelILi512ELb1ELb0ELb0ELi4EEEvNS_6ParamsEi"),
     # the decode step's output projection and the prompt's head transform
     ("output_block.hip", "_ZN3pcl22project_row_lds_kernelENS_11BlockParamsEi"),
+    ("output_block.hip", "_ZN3pcl19project_rows_kernelILi5EEEvNS_11BlockParamsE"),
+    ("output_block.hip", "_ZN3pcl18project_few_kernelILi1EEEvNS_11BlockParamsE"),
+    ("output_block.hip", "_ZN3pcl18project_few_kernelILi2EEEvNS_11BlockParamsE"),
+    ("output_block.hip", "_ZN3pcl20project_tiles_kernelILi128ELi128ELi32EEEvNS_11BlockParamsE"),
+    ("output_block.hip", "_ZN3pcl20project_tiles_kernelILi32ELi32ELi128EEEvNS_11BlockParamsE"),
     ("head_transform.hip", "_ZN3pcl21head_transform_kernelILi256ELi16EEEvNS_15TransformParamsE"),
     ("head_transform.hip", "_ZN3pcl21head_transform_kernelILi512ELi8EEEvNS_15TransformParamsE"),
 ])
