@@ -129,3 +129,46 @@ def test_capture_refuses_an_explicit_spread_request(pcl, torch):
         assert np.array_equal(bits(got), bits(want))
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 4, 20, 40, 200, 700, 1400])
+def test_output_block_replays_give_the_eager_bits(pcl, torch, n):
+    # every projection form, captured without an eager call on its stream
+    cols, rows = 516, 2816
+    dev = torch.device("cuda:0")
+    stream = torch.cuda.Stream()
+    ctx = pcl.Context(0, stream.cuda_stream)
+    plain = pcl.Context(0, torch.cuda.current_stream().cuda_stream)
+    try:
+        x, res = torch.empty((n, cols), device=dev), torch.empty((n, rows), device=dev)
+        w = torch.randn((rows, cols), device=dev)
+        scale = torch.randn(rows, device=dev)
+        proj, out = torch.empty((n, rows), device=dev), torch.empty((n, rows), device=dev)
+
+        def call(c, p, o):
+            c.attention_output(x.data_ptr(), n, cols, w.data_ptr(), rows, scale.data_ptr(), 1e-6,
+                               res.data_ptr(), p.data_ptr(), o.data_ptr())
+
+        x.normal_()
+        res.normal_()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call(ctx, proj, out)
+        for _ in range(4):
+            x.normal_()
+            res.normal_()
+            proj.fill_(float("nan"))
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            want_p, want = torch.empty_like(proj), torch.empty_like(out)
+            call(plain, want_p, want)
+            assert plain.sync() == 0 and ctx.sync() == 0
+            assert np.array_equal(bits(proj.cpu().numpy()), bits(want_p.cpu().numpy()))
+            assert np.array_equal(bits(out.cpu().numpy()), bits(want.cpu().numpy()))
+        graph.reset()
+    finally:
+        ctx.close()
+        plain.close()
