@@ -449,8 +449,8 @@ int pcl_attention_output(pcl_context *ctx, const float *attended, int64_t n, int
 
 /* For tests: which form of the projection n tokens of `in` columns take on a
  * device of `cus` compute units: 1 a wave per output row, 16 or 32 the
- * few-token kernel with so many tokens a workgroup, else the output tile's
- * tokens * 1000 + rows. */
+ * few-token kernel with so many tokens a workgroup, else the output block of
+ * a wave (16016) or tile of a workgroup as tokens * 1000 + rows. */
 int pcl_debug_projection_form(int64_t n, int64_t in, int64_t out, int cus);
 
 /* Library identification (for loaders). */

@@ -10,7 +10,7 @@
 // the two f64 sums straddle an f32 rounding boundary, and a sum like
 // 2^24 + 1 - 2^24 stays exact. The order depends on the token count only: one
 // for up to 32 tokens (the first three kernels give the same bits), one for
-// more (the tiles of every shape).
+// more (the chains and the tiles of every shape).
 //
 //   project_rows_kernel: up to five tokens. HBM-bound on the
 //     weights: one wave per output row streams the row once with 16-byte
@@ -23,6 +23,8 @@
 //   project_few_kernel: up to 32 tokens (verification, short prompts): the
 //     waves of a workgroup split the columns of 16 output rows, f64 MFMAs on
 //     operands loaded straight from memory.
+//   project_chain_kernel: more tokens, while 16 x 16 blocks are one per SIMD:
+//     f64 MFMAs on operands loaded straight from memory, one chain a wave.
 //   project_tiles_kernel: more tokens (prompt). MFMA-bound: output
 //     tiles of 128 x 128 down to 32 x 32, K steps double-buffered in LDS as
 //     f32, the products on v_mfma_f64_16x16x4f64 after converting the
@@ -646,6 +648,91 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void project_few_kernel(BlockPar
     }
 }
 
+// 16 output rows x 16 tokens per wave, a workgroup of its own: one f64 MFMA
+// chain over the columns in the order of the tiles (the same bits), operands
+// loaded straight from memory kChainAhead groups of 16 columns ahead and
+// converted one group ahead (a conversion into registers that an MFMA still
+// reads waits for it). No LDS and no barriers, and up to 1024 blocks run one
+// chain per SIMD.
+constexpr int kChainAhead = 12;
+
+__global__ __launch_bounds__(64) void project_chain_kernel(BlockParams p, int blocks)
+{
+    const int lane = threadIdx.x;
+    const int r16 = lane & 15, kq = lane >> 4;
+    // consecutive workgroups go to the 8 XCDs in turn: a row group's token
+    // blocks take one XCD, whose L2 then serves its weights
+    const int slot = blockIdx.x / 8;
+    const int r0 = (slot / blocks * 8 + blockIdx.x % 8) * 16, t0 = slot % blocks * 16;
+    if (r0 >= p.out)
+        return;
+    // rows and tokens past the last repeat it (not written)
+    const float *wr = p.w + (int64_t)min(r0 + r16, p.out - 1) * p.in + 4 * kq;
+    const float *xr = p.x + (int64_t)min(t0 + r16, p.n - 1) * p.in + 4 * kq;
+    const int groups = p.in / 16;
+
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    double cx[2][4], cw[2][4];
+    auto convert = [&](const f4 &x, const f4 &w, int set) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            cx[set][j] = (double)x[j];
+            cw[set][j] = (double)w[j];
+        }
+    };
+    // MFMA k slot kq of step j holds column 16 g + 4 kq + j
+    auto multiply = [&](int set) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(cx[set][j], cw[set][j], acc, 0, 0, 0);
+    };
+    if (groups > 0) {
+        f4 x[kChainAhead], w[kChainAhead];
+        // a group past the last whole one repeats it (not multiplied)
+        auto load = [&](int g, int d) {
+            const int at = 16 * min(g, groups - 1);
+            x[d] = ldg4(xr + at);
+            w[d] = ldg4(wr + at);
+        };
+#pragma unroll
+        for (int d = 0; d < kChainAhead; ++d)
+            load(d, d);
+        convert(x[0], w[0], 0);
+        static_assert(kChainAhead % 2 == 0, "a group's operand set by its place in the loop");
+        for (int g = 0; g < groups; g += kChainAhead) {
+#pragma unroll
+            for (int d = 0; d < kChainAhead; ++d) {
+                if (g + d < groups) {
+                    load(g + d + kChainAhead, d);
+                    __builtin_amdgcn_sched_barrier(0);
+                    convert(x[(d + 1) % kChainAhead], w[(d + 1) % kChainAhead], (d + 1) & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    multiply(d & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+    }
+    if (p.in % 16) {
+        f4 x, w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool in = 16 * groups + 4 * kq + e < p.in;
+            x[e] = in ? ldg(xr + 16 * groups + e) : 0.f;
+            w[e] = in ? ldg(wr + 16 * groups + e) : 0.f;
+        }
+        convert(x, w, 0);
+        multiply(0);
+    }
+    // element e: token kq + 4e, row r16
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int t = t0 + kq + 4 * e, r = r0 + r16;
+        if (t < p.n && r < p.out)
+            stg(p.proj + (int64_t)t * p.out + r, (float)acc[e]);
+    }
+}
+
 template <int TM, int TN, int TK>
 static hipError_t launch_tile(const BlockParams &p, hipStream_t stream)
 {
@@ -729,6 +816,20 @@ static int few_blocks(int64_t n, int64_t out, int64_t cus)
     return blocks == 1 || blocks * ((out + 15) / 16) <= cus ? 1 : 2;
 }
 
+// Whether project_chain_kernel takes n tokens: up to 128 of them while every
+// 16 x 16 block is the only chain of its SIMD. Its time is then the chain's,
+// where the tiles' K steps add theirs: 2816 x 4096, 33 tokens 45.9 us against
+// 51.9 us in tiles, 64 tokens 51.7 and 52.0 us, 80 tokens 64.3 and 83.9 us; 96
+// tokens, where some SIMDs take two chains, 88 against 84 us. More tokens of
+// few rows crowd the few XCDs that have a row group (1024 -> 300, 800 tokens:
+// 29.4 against 22.8 us).
+constexpr int kChainTo = 128;
+
+static bool chain_fits(int64_t n, int64_t out, int64_t cus)
+{
+    return n <= kChainTo && (n + 15) / 16 * ((out + 15) / 16) <= 4 * cus;
+}
+
 hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
 {
     const int cus = std::max(device_cus(), 1);
@@ -752,6 +853,9 @@ hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)
             project_few_kernel<1><<<dim3(rows, (p.n + 15) / 16), 64 * kFewWaves, 0, stream>>>(p);
         else
             project_few_kernel<2><<<rows, 64 * kFewWaves, 0, stream>>>(p);
+    } else if (chain_fits(p.n, p.out, cus)) {
+        const int rows = (p.out + 15) / 16, blocks = (p.n + 15) / 16;
+        project_chain_kernel<<<(rows + 7) / 8 * 8 * blocks, 64, 0, stream>>>(p, blocks);
     } else {
         const hipError_t e = choose_tile(p.n, p.in, p.out, cus).launch(p, stream);
         if (e != hipSuccess)
@@ -802,6 +906,8 @@ extern "C" int pcl_debug_projection_form(int64_t n, int64_t in, int64_t out, int
         return 1;
     if (n <= pcl::kFewTo)
         return 16 * pcl::few_blocks(n, out, cus);
+    if (pcl::chain_fits(n, out, std::max(cus, 1)))
+        return 16016;
     const pcl::Tile &t = pcl::choose_tile(n, in, out, std::max(cus, 1));
     return 1000 * t.m + t.n;
 }

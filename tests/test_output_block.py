@@ -79,7 +79,7 @@ def run_block(torch, ctx, x, w, scale, res, eps=1e-6, in_place=False):
 
 
 # n = 1 and 5: a wave per output row; 7, 16, 17, 32: the few-token kernel; 33,
-# 200, 300: f64 MFMA tiles. One token
+# 200, 300: a wave per 16 x 16 block. One token
 # with input rows of at most 16384 columns (a multiple of 4) is projected
 # with the input row staged in LDS: rows of 1000 (fewer than 4096 columns),
 # 5000 (4096 and a partial step), 4000 (one 4096-column step taken by some
@@ -114,24 +114,25 @@ def test_output_block_matches_the_oracle(torch, ctx, oracle, case):
 
 
 # (tokens, columns, output rows) and the form they take on 256 CUs: a wave per
-# output row (1), the few-token kernel with 16 or 32 tokens a workgroup, or
-# output tiles of tokens x rows (tokens * 1000 + rows). Per tile shape: a
-# remainder of tokens and rows, columns below one K step, and more than two K
-# steps with a remainder. The few-token kernel: one to 32 tokens around its
-# blocks of 16, output rows of 16 and one past, columns within one wave's 16,
-# at and past 256-column steps, and remainders of a quad; enough rows for
-# two blocks a workgroup.
+# output row (1), the few-token kernel with 16 or 32 tokens a workgroup, a
+# wave per 16 x 16 block (16016: columns below, at and past its groups of 16
+# and its 12 groups in flight), or output tiles of tokens x rows (tokens *
+# 1000 + rows). Per tile shape: a remainder of tokens and rows, columns below
+# one K step, and more than two K steps with a remainder. The few-token
+# kernel: one to 32 tokens around its blocks of 16, output rows of 16 and one
+# past, columns within one wave's 16, at and past 256-column steps, and
+# remainders of a quad; enough rows for two blocks a workgroup.
 FORMS = {
     (3, 4, 1): 1, (4, 28, 16): 1, (5, 4096, 2816): 1, (3, 1001, 77): 1, (5, 1003, 33): 1,
     (6, 4, 1): 16, (13, 1001, 77): 16, (16, 260, 17): 16, (17, 256, 33): 16, (31, 126, 32): 16,
     (17, 127, 33): 16, (32, 516, 16): 16, (31, 770, 4100): 32, (32, 1024, 2816): 32,
-    (33, 512, 40): 32032, (40, 130, 65): 32032, (64, 1028, 31): 32032, (65, 772, 33): 32032,
-    (128, 96, 18): 32032, (129, 68, 2816): 32032, (200, 381, 2816): 32032,
+    (33, 3, 17): 16016, (33, 512, 40): 16016, (40, 130, 65): 16016, (48, 16, 129): 16016,
+    (64, 1028, 31): 16016, (65, 772, 33): 16016, (80, 209, 2816): 16016, (128, 96, 18): 16016,
+    (81, 381, 2811): 32032, (129, 68, 2816): 32032, (200, 381, 2816): 32032, (65, 96, 4220): 32032,
     (530, 34, 4220): 64032, (480, 200, 2816): 64032, (497, 261, 2801): 64032,
-    (65, 96, 4220): 32032,
     (700, 63, 2816): 64064, (700, 330, 2816): 64064, (300, 199, 2803): 64064,
-    (520, 65, 2816): 128064, (2100, 101, 2816): 128064,
-    (1400, 31, 2816): 128128, (1400, 133, 2816): 128128, (1301, 98, 2790): 128128,
+    (520, 65, 2816): 128064, (2100, 101, 2816): 128064, (1400, 31, 2816): 128128,
+    (1400, 133, 2816): 128128, (1301, 98, 2790): 128128,
 }
 
 
@@ -145,6 +146,8 @@ def test_projection_forms(pcl):
     assert form(2000, 96, 2816, 256) == 128064 and form(2000, 4096, 2816, 256) == 64032
     assert form(520, 64, 2816, 256) in (64064, 64032, 128064)
     assert form(1, 4096, 2816, 256) == 1 and form(33, 4096, 2816, 0) // 1000 >= 32
+    # one chain per SIMD, or tiles
+    assert form(80, 4096, 2816, 256) == 16016 and form(81, 4096, 2816, 256) == 32032
     # sizes at the entry's limits stay within a grid's 65535 blocks of rows
     assert form(1 << 22, 1 << 20, 1 << 20, 256) == 128128
     for n, out in ((1 << 22, 16), (1 << 22, 1 << 20), (1 << 20, 128)):
@@ -201,10 +204,10 @@ def test_one_token_projection_equals_the_multi_token_one_bitwise(torch, ctx, col
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", [(3, 4096, 300), (2, 1001, 33), (4, 1000, 300), (5, 8193, 16),
                                   (6, 1028, 33), (8, 4098, 17), (16, 260, 64), (16, 1, 1),
-                                  (17, 4096, 130), (31, 1003, 48), (32, 512, 4200), (17, 259, 2816), (32, 3, 4200),
-                                  (34, 4097, 33), (64, 1028, 300), (128, 196, 65),
-                                  (200, 1000, 2816), (480, 200, 2816), (520, 515, 2816),
-                                  (700, 261, 2816),
+                                  (17, 4096, 130), (31, 1003, 48), (32, 512, 4200),
+                                  (17, 259, 2816), (32, 3, 4200), (34, 4097, 33), (64, 1028, 300),
+                                  (128, 196, 65), (96, 260, 2816), (200, 1000, 2816),
+                                  (480, 200, 2816), (520, 515, 2816), (700, 261, 2816),
                                   (1400, 133, 2816), (2100, 130, 2816)],
                          ids=lambda c: "x".join(map(str, c)))
 def test_a_tokens_projection_does_not_depend_on_the_token_count(torch, ctx, case):
