@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
     // global -> registers -> LDS; the next step's loads are in flight during
     // this step's MFMAs. Rows past the last repeat it (not written), columns
     // past the last are zero: a branch around each load of a whole step cost
-    // 6 to 16 % (64 tokens of 4096 columns 69 -> 60 us, 2000 tokens 866 -> 791).
+    // 6 to 16 % (256 tokens of 4096 columns 159 -> 142 us, 2000 tokens 866 -> 791).
     f4 ra[kLoadA], rb[kLoadB];
     auto load = [&](int k0) {
         if (k0 + TK <= p.in) { // all loads go out together
@@ -233,8 +233,8 @@ __global__ __launch_bounds__(256, 2) void project_tiles_kernel(BlockParams p)
             // A single chain of MFMAs: each would wait for its operands'
             // conversions, and these for the MFMA before it that still reads
             // their registers. Operands are read 32 and converted 16 columns
-            // ahead into registers of their own (64 tokens of 4096 columns,
-            // 2816 rows: 57.8 -> 52.5 us).
+            // ahead into registers of their own (256 tokens of 4096 columns, 2816
+            // rows: 135.7 -> 125.7 us; 64 tokens 57.8 -> 52.5 us).
             const float *ar = sa + (buf * TM + wm + r16) * kRow + 4 * kq;
             const float *br = sb + (buf * TN + wn + r16) * kRow + 4 * kq;
             f4 a[2], b[2];
@@ -779,8 +779,8 @@ constexpr Tile kTiles[] = {
 // CUs idle under large tiles, while small ones reach a lower MFMA rate. Of 224
 // sizes timed in every shape the choice is 0.6 % from the best on average.
 // Projection of 2816 rows of 4096 columns, 128 x 128 alone (its loads
-// branching over rows and columns) against the chosen tile: 33 tokens 568 ->
-// 53 us, 256 tokens 581 -> 126 us, 1000 tokens 589 -> 421 us, 2000 tokens 1076
+// branching over rows and columns) against the chosen tile: 100 tokens 577 ->
+// 85 us, 256 tokens 581 -> 126 us, 1000 tokens 589 -> 421 us, 2000 tokens 1076
 // -> 783 us, 4096 tokens 1.62 -> 1.49 ms (0.81 of the fp64 MFMA peak); 2000
 // tokens of 96 columns 44 -> 38 us (49 us by a rule without the column count).
 static const Tile &choose_tile(int64_t n, int64_t in, int64_t out, int64_t cus)
