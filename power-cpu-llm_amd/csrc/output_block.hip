@@ -469,7 +469,10 @@ __device__ __forceinline__ f4 transpose_groups(f4 v)
 // 16 output rows x 16 NB tokens per workgroup, its eight waves splitting the
 // columns. A wave loads MFMA operands straight from memory (every weight is
 // used by one wave only, so LDS would add a pass), the next 256 columns'
-// requested ahead of the ones being multiplied.
+// requested ahead of the ones being multiplied. Two waves share a 128-byte
+// line of the weights, so these are plain loads: streaming ones took 37.9
+// against 35.6 us at 8 tokens of 8192 columns, 2816 rows from HBM (25.2 against
+// 21.9 us at 16 tokens of 4096 columns from the last-level cache).
 //
 // Every output is the sum that project_rows_kernel forms, bit for bit, so a
 // token's row does not depend on how many tokens come with it: that kernel's
@@ -481,12 +484,10 @@ __device__ __forceinline__ f4 transpose_groups(f4 v)
 // wave, 16, 8 and 4 with other waves through LDS, 2 and 1 in the wave.
 //
 // Bound by the weights' stream and its round trips, at 32 tokens also by the
-// MFMAs of the CUs that have a group of rows (13.7 us of the 35 at 4096
-// columns, at the fp64 peak). 2816 x 4096 with its post-norm, one wave per row against
-// this: 8 tokens 33.2 -> 21.4 us, 16 tokens 52 -> 25.3 us, 32 tokens 117 ->
-// 35.2 us. Eight accumulators a token block of the wave, the transposes and
-// the exchange cost 0.6 to 3.5 us of it against sums in whatever order is
-// nearest (16 tokens 24.2, 32 tokens 31.8 us).
+// MFMAs of the CUs that have a group of rows (13.7 us of the 31 at 4096
+// columns, at the fp64 peak). 2816 x 4096 with its post-norm, one wave per row
+// against this: 8 tokens 33.2 -> 19.5 us, 16 tokens 52 -> 21.9 us, 32 tokens
+// 117 -> 31.4 us (from HBM 21.3, 25.1 and 34.8 us).
 constexpr int kFewWaves = 8;
 constexpr int kFewStep = 256; // columns per step: one quad of every lane sum
 
@@ -519,7 +520,7 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void project_few_kernel(BlockPar
         for (int h = 0; h < 2; ++h) {
             const int c = k + c0 + 128 * h;
             const int at = c < whole ? c : 0;
-            v.w[h] = ldg4_stream(wr + at);
+            v.w[h] = ldg4(wr + at);
 #pragma unroll
             for (int b = 0; b < NB; ++b)
                 v.x[b][h] = ldg4(xr[b] + at);
@@ -654,7 +655,7 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void project_few_kernel(BlockPar
 // converted one group ahead (a conversion into registers that an MFMA still
 // reads waits for it). No LDS and no barriers, and up to 1024 blocks run one
 // chain per SIMD.
-constexpr int kChainAhead = 12;
+constexpr int kChainAhead = 16;
 
 __global__ __launch_bounds__(64) void project_chain_kernel(BlockParams p, int blocks)
 {
@@ -802,7 +803,7 @@ static const Tile &choose_tile(int64_t n, int64_t in, int64_t out, int64_t cus)
 // Tokens project_few_kernel takes: from 6 (one wave per row spreads over more
 // CUs; 3 tokens 8192 -> 5376 rows of weights 59.7 us there and 71.6 us here,
 // 16384 -> 1024 34.0 and 55.8 us, 4096 -> 2816 17.7 and 19.5 us; 5 tokens 4096
-// -> 2816 19.8 and 20.0 us; 6 tokens 25.8 and 20.4 us) up to the 32 that two
+// -> 2816 19.8 and 20.0 us; 6 tokens 25.8 and 19.3 us) up to the 32 that two
 // 16-token blocks of a workgroup hold. Past 16 tokens each workgroup takes
 // both (the weights are read once) unless single blocks fit one round of the
 // CUs (2048 x 2048, 32 tokens: 15.5 us in single blocks, 19.0 us in pairs;
@@ -818,16 +819,20 @@ static int few_blocks(int64_t n, int64_t out, int64_t cus)
 
 // Whether project_chain_kernel takes n tokens: up to 128 of them while every
 // 16 x 16 block is the only chain of its SIMD. Its time is then the chain's,
-// where the tiles' K steps add theirs: 2816 x 4096, 33 tokens 45.9 us against
-// 51.9 us in tiles, 64 tokens 51.7 and 52.0 us, 80 tokens 64.3 and 83.9 us; 96
-// tokens, where some SIMDs take two chains, 88 against 84 us. More tokens of
-// few rows crowd the few XCDs that have a row group (1024 -> 300, 800 tokens:
-// 29.4 against 22.8 us).
+// where the tiles' K steps add theirs and a half-empty tile of 32 tokens its
+// own: 2816 x 4096, weights from HBM, 33 tokens 48.8 us against 52.4 us in tiles
+// of 32 x 32, 80 tokens 72 against 85 us; 96 tokens, where some SIMDs take two
+// chains, 88 against 84 us (from the last-level cache). Full tiles on more
+// than half of the CUs read the weights once for two chains: 64 tokens 55.9
+// against 52.1 us. More tokens of few rows crowd the few XCDs that have a row
+// group (1024 -> 300, 800 tokens: 29.4 against 22.8 us).
 constexpr int kChainTo = 128;
 
 static bool chain_fits(int64_t n, int64_t out, int64_t cus)
 {
-    return n <= kChainTo && (n + 15) / 16 * ((out + 15) / 16) <= 4 * cus;
+    const int64_t blocks = (n + 15) / 16;
+    const bool full_tiles = blocks % 2 == 0 && 2 * (blocks / 2 * ((out + 31) / 32)) > cus;
+    return n <= kChainTo && blocks * ((out + 15) / 16) <= 4 * cus && !full_tiles;
 }
 
 hipError_t launch_output_block(const BlockParams &p, hipStream_t stream)

@@ -116,7 +116,7 @@ def test_output_block_matches_the_oracle(torch, ctx, oracle, case):
 # (tokens, columns, output rows) and the form they take on 256 CUs: a wave per
 # output row (1), the few-token kernel with 16 or 32 tokens a workgroup, a
 # wave per 16 x 16 block (16016: columns below, at and past its groups of 16
-# and its 12 groups in flight), or output tiles of tokens x rows (tokens *
+# and its 16 groups in flight), or output tiles of tokens x rows (tokens *
 # 1000 + rows). Per tile shape: a remainder of tokens and rows, columns below
 # one K step, and more than two K steps with a remainder. The few-token
 # kernel: one to 32 tokens around its blocks of 16, output rows of 16 and one
@@ -127,7 +127,7 @@ FORMS = {
     (6, 4, 1): 16, (13, 1001, 77): 16, (16, 260, 17): 16, (17, 256, 33): 16, (31, 126, 32): 16,
     (17, 127, 33): 16, (32, 516, 16): 16, (31, 770, 4100): 32, (32, 1024, 2816): 32,
     (33, 3, 17): 16016, (33, 512, 40): 16016, (40, 130, 65): 16016, (48, 16, 129): 16016,
-    (64, 1028, 31): 16016, (65, 772, 33): 16016, (80, 209, 2816): 16016, (128, 96, 18): 16016,
+    (64, 1028, 31): 16016, (65, 772, 33): 16016, (80, 277, 2816): 16016, (128, 96, 18): 16016,
     (81, 381, 2811): 32032, (129, 68, 2816): 32032, (200, 381, 2816): 32032, (65, 96, 4220): 32032,
     (530, 34, 4220): 64032, (480, 200, 2816): 64032, (497, 261, 2801): 64032,
     (700, 63, 2816): 64064, (700, 330, 2816): 64064, (300, 199, 2803): 64064,
@@ -148,6 +148,7 @@ def test_projection_forms(pcl):
     assert form(1, 4096, 2816, 256) == 1 and form(33, 4096, 2816, 0) // 1000 >= 32
     # one chain per SIMD, or tiles
     assert form(80, 4096, 2816, 256) == 16016 and form(81, 4096, 2816, 256) == 32032
+    assert form(48, 4096, 2816, 256) == 16016 and form(64, 4096, 2816, 256) == 32032
     # sizes at the entry's limits stay within a grid's 65535 blocks of rows
     assert form(1 << 22, 1 << 20, 1 << 20, 256) == 128128
     for n, out in ((1 << 22, 16), (1 << 22, 1 << 20), (1 << 20, 128)):
