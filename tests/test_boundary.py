@@ -277,6 +277,7 @@ def _resource_remarks(source):
     ("output_block.hip", "_ZN3pcl19project_rows_kernelILi5EEEvNS_11BlockParamsE"),
     ("output_block.hip", "_ZN3pcl18project_few_kernelILi1EEEvNS_11BlockParamsE"),
     ("output_block.hip", "_ZN3pcl18project_few_kernelILi2EEEvNS_11BlockParamsE"),
+    ("output_block.hip", "_ZN3pcl20project_chain_kernelENS_11BlockParamsEi"),
     ("output_block.hip", "_ZN3pcl20project_tiles_kernelILi128ELi128ELi32EEEvNS_11BlockParamsE"),
     ("output_block.hip", "_ZN3pcl20project_tiles_kernelILi32ELi32ELi128EEEvNS_11BlockParamsE"),
     ("head_transform.hip", "_ZN3pcl21head_transform_kernelILi256ELi16EEEvNS_15TransformParamsE"),
